@@ -36,11 +36,16 @@ ELEM_TYPES = {"rectangle": 1, "triangle": 2, "ellipse": 3, "sector": 4, "segment
 GEOMETRY_IDS = {"parallel": 0, "equiangular": 1, "equilinear": 2}
 
 
+def have_ref_sources() -> bool:
+    """Whether the reference's sources are there (its folder may be empty)."""
+    return os.path.isdir(os.path.join(REF_SRC, "libctsim"))
+
+
 def build(ref: bool | None = None) -> None:
     """Compile liboracle.so, and the reference library when its sources exist."""
     subprocess.check_call(["make", "-s", "-C", HERE, "oracle"])
     if ref is None:
-        ref = os.path.isdir(REF_SRC)
+        ref = have_ref_sources()
     if ref:
         subprocess.check_call(["make", "-s", "-j8", "-C", HERE, "ref", f"REF={REF_SRC}"])
 
