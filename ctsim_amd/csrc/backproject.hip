@@ -628,9 +628,13 @@ int view_consts(ctsim_ctx* ctx, const BpPlan& p, int kind, const double* h_angle
 int bp_upload_tables(BpPlan& p) {
   if (!p.r.empty()) {
     size_t n = p.r.size();
-    CTSIM_CHECK(p.d_rphi.reserve(2 * n * sizeof(double)));
+    CTSIM_CHECK(p.d_rphi.reserve((2 * n + p.nx + p.ny) * sizeof(double)));
     CTSIM_HIP(hipMemcpy(p.d_rphi.ptr, p.r.data(), n * sizeof(double), hipMemcpyHostToDevice));
     CTSIM_HIP(hipMemcpy(p.d_rphi.as<double>() + n, p.phi.data(), n * sizeof(double),
+                        hipMemcpyHostToDevice));
+    std::vector<double> xy(p.xd);
+    xy.insert(xy.end(), p.yd.begin(), p.yd.end());
+    CTSIM_HIP(hipMemcpy(p.d_rphi.as<double>() + 2 * n, xy.data(), xy.size() * sizeof(double),
                         hipMemcpyHostToDevice));
   }
   CTSIM_CHECK(p.d_xy.reserve((p.xs.size() + p.ys.size()) * sizeof(float)));
@@ -672,7 +676,18 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
   if (f64) {
     CTSIM_CHECK(view_consts<ViewConstF64>(
         ctx, p, 0, h_angles, nView,
-        [&](ViewConstF64* o) { bp_view_consts_f64(p, h_angles, nView, o); }, &a.vc));
+        [&](ViewConstF64* o) {
+          bp_view_consts_f64(p, h_angles, nView, o);
+          p.cachedMaxAngle = 0;
+          for (int v = 0; v < nView; v++) {
+            const double m = fabs(h_angles[v]);
+            if (!(m <= p.cachedMaxAngle)) p.cachedMaxAngle = m;  // (a NaN stays)
+          }
+        },
+        &a.vc));
+    if (!inF32 && bp_fan_f64_ok(p, p.cachedMaxAngle))
+      return bp_fan_f64_launch(ctx, p, static_cast<const double*>(d_filtered),
+                               static_cast<const ViewConstF64*>(a.vc), nView, d_image);
     if (p.kind == KIND_DIFF) {
       const int g = (p.nx + 63) / 64;
       if (inF32) launch_diff<float>(p.interp, a, g, s);

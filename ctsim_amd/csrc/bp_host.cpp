@@ -135,13 +135,15 @@ int bp_plan_init(BpPlan& p, int geometry, int nDet, double detInc, int nView,
   p.sdl = sdl;
 
   // Pixel-centre tables by repeated addition (backprojectors.cpp:374-377, 424-428).
-  p.xs.resize(nx);
-  p.ys.resize(ny);
+  p.xd.resize(nx);
+  p.yd.resize(ny);
   {
     double x = p.xMin + p.xInc / 2;
-    for (int ix = 0; ix < nx; x += p.xInc, ix++) p.xs[ix] = static_cast<float>(x);
+    for (int ix = 0; ix < nx; x += p.xInc, ix++) p.xd[ix] = x;
     double y = p.yMin + p.yInc / 2;
-    for (int iy = 0; iy < ny; y += p.yInc, iy++) p.ys[iy] = static_cast<float>(y);
+    for (int iy = 0; iy < ny; y += p.yInc, iy++) p.yd[iy] = y;
+    p.xs.assign(p.xd.begin(), p.xd.end());
+    p.ys.assign(p.yd.begin(), p.yd.end());
   }
   if (p.kind == KIND_TRIG || p.kind == KIND_TABLE || p.kind == KIND_EQUIANGULAR ||
       p.kind == KIND_EQUILINEAR) {
@@ -242,6 +244,9 @@ void bp_view_consts_f64(const BpPlan& p, const double* angles, int nView, ViewCo
       memcpy(&c.a, &dx, 8);
       memcpy(&c.b, &dy, 8);
       memcpy(&c.c, &cs, 8);
+    } else if (p.geom != GEOM_PARALLEL) {
+      c.a = cos(theta);
+      c.b = sin(theta);
     }
   }
 }

@@ -21,6 +21,7 @@ enum BpKind {
 struct ViewConstF64 {
   double theta;     // view angle (Trig, Table, fan)
   double a, b;      // Diff: det_dx, det_dy       IntDiff: bit patterns of int64 det_dx, det_dy
+                    // fan: cos, sin of theta
   double c;         // Diff: detPosColStart       IntDiff: bit pattern of int64 colStart
 };
 
@@ -85,9 +86,10 @@ struct BpPlan {
   double F = 0, sdl = 0, start_r = 0, start_phi = 0, viewDiameter = 0;
   // Host tables (built exactly as the reference builds them).
   std::vector<double> r, phi;       // [nx*ny] column-major, Table/fan/Trig
-  std::vector<float> xs, ys;        // pixel-centre coordinates (mixed path)
+  std::vector<double> xd, yd;       // pixel-centre coordinates (repeated additions)
+  std::vector<float> xs, ys;        // the same rounded to float (mixed path)
   // Device copies.
-  DevBuf d_rphi;                    // r then phi, doubles
+  DevBuf d_rphi;                    // r, phi, xd, yd, doubles
   DevBuf d_xy;                      // xs then ys, floats
   // Launch shape.
   int tileX = 16, tileY = 16;       // pixels per block along ix, iy
@@ -111,6 +113,7 @@ struct BpPlan {
   mutable int cachedKind = -1;      // 0: FP64 constants, 1: FP32 constants
   mutable DevBuf d_vc;
   mutable SymViews cachedSym;       // symmetry of the cached angles (FP32 constants)
+  mutable double cachedMaxAngle = 0;  // largest |angle| of the cached angles (FP64 constants)
 };
 
 // Host side (bp_host.cpp).
@@ -144,6 +147,12 @@ int bp_mixed_tiles(ctsim_ctx* ctx, const BpPlan& p, const MixedShape& m, const v
                    bool overwrite, const SymViews* views = nullptr, float* partial = nullptr);
 int bp_view_consts_mixed(ctsim_ctx* ctx, const BpPlan& p, const double* h_angles, int nView,
                          const ViewConstF32** out);
+// The fan-beam FP64 kernel with linear or cubic interpolation
+// (backproject_f64.hip): whether its error bounds cover this plan and view
+// angles up to maxAngle in size, and its launch over nView filtered rows.
+bool bp_fan_f64_ok(const BpPlan& p, double maxAngle);
+int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
+                      int nView, float* d_image);
 // True when the mixed precision of this plan runs the tiled coefficient
 // kernel (not the FP64 index path) and one view's staging fits LDS.
 bool bp_mixed_tiled(const BpPlan& p);
