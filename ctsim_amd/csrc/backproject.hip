@@ -688,6 +688,9 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
     if (!inF32 && bp_fan_f64_ok(p, p.cachedMaxAngle))
       return bp_fan_f64_launch(ctx, p, static_cast<const double*>(d_filtered),
                                static_cast<const ViewConstF64*>(a.vc), nView, d_image);
+    if (!inF32 && bp_idiff_f64_ok(p))
+      return bp_idiff_f64_launch(ctx, p, static_cast<const double*>(d_filtered),
+                                 static_cast<const ViewConstF64*>(a.vc), nView, d_image);
     if (p.kind == KIND_DIFF) {
       const int g = (p.nx + 63) / 64;
       if (inF32) launch_diff<float>(p.interp, a, g, s);

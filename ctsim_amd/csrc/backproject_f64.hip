@@ -1,5 +1,7 @@
-// FP64 fan-beam backprojection for gfx950, linear and cubic interpolation.
+// FP64 fan-beam and IntDiff backprojection for gfx950, linear and cubic
+// interpolation.
 //
+// Fan beam.
 // The reference adds every view's contribution to a float32 pixel,
 // v = float(double(v) + c) (backprojectors.cpp:656-743), with c built from a
 // cosine, a sine, an arc tangent and divisions, each rounded in its own
@@ -416,6 +418,219 @@ void launch_fan_kind(const BpPlan& p, int deg, const FanF64Args& a, int grid, si
   else launch_fan<KIND_EQUIANGULAR, INTERP, kMaxDeg>(a, grid, lds, s);
 }
 
+// ------------------------------------------------------------------ IntDiff
+
+// BackprojectIntDiff (backprojectors.cpp:579-653) walks the image in 32.32
+// fixed point.  Every such position is a whole multiple of 2^-32 and, below
+// 2^20 cells, an FP64 number: the positions are formed exactly in FP64, the
+// interval and the fraction are the fixed-point ones, and scaling the slope by
+// 2^-32 and the remainder by 2^32, as the reference does, changes no rounding.
+// Linear interpolation then does the reference's own two operations; cubic
+// interpolation evaluates the interval's polynomial, within kCubicRound of the
+// largest cell of the reference's Lagrange sum, and decides the float32 sum as
+// the fan-beam kernel does.  Outside the detector the linear coefficients are
+// -0.0, which leaves any v as it is (the reference skips the sample), the
+// cubic ones 0.0, which the reference adds.
+//
+// What bounds it: FP64 VALU issue.  2048^2 pixels, 2880 views, linear: 37.4
+// lane instructions per update and 15.1 ms with the fixed-point walk of one
+// pixel per lane, about 12 and 4.5 ms here (56 cycles per wave and update, 12
+// instructions at the 4.7 cycles that an FP64 instruction takes on this chip);
+// 256^2, 320 views: 184 us and 27.
+struct IdiffArgs {
+  int nx, ny, nDet, nView;
+  int tilesY, W, views, half;  // views: staged at a time; half: 32 lanes stage a window
+  const double* f;
+  const ViewConstF64* vc;
+  float* image;
+};
+
+// the reference's Lagrange sum and the staged polynomial (40 u, as in
+// fan_bounds), and a quarter more
+constexpr double kCubicRound = 1.25 * 40 * 0x1p-53;
+
+template <int INTERP>
+struct IdiffCell {  // the line's value and slope, or the cubic's coefficients and rounding bound
+  double v[INTERP == INTERP_CUBIC ? 6 : 2];
+};
+
+template <int INTERP>
+__device__ __forceinline__ void idiff_coef(double y0, double y1, double y2, double y3, int i, int n,
+                                           IdiffCell<INTERP>* cell) {
+  double2* out = reinterpret_cast<double2*>(cell->v);
+  if constexpr (INTERP == INTERP_LINEAR) {
+    const bool in = i >= 0 && i < n;  // the last cell's value is held
+    out[0] = make_double2(in ? y1 : -0.0, in ? (i < n - 1 ? y2 - y1 : 0.0) : -0.0);
+  } else {
+    const double third = 1. / 3, sixth = 1. / 6;
+    const bool in = i >= 0 && i + 2 <= n, interior = i > 0 && i + 2 < n;  // else (in) the end intervals: a line
+    const double b1 = fma(-third, y0, fma(-0.5, y1, fma(-sixth, y3, y2)));
+    const double b2 = fma(0.5, y0 + y2, -y1);
+    const double b3 = fma(sixth, y3 - y0, 0.5 * (y1 - y2));
+    const double big = fmax(fmax(fabs(y0), fabs(y1)), fmax(fabs(y2), fabs(y3)));
+    out[0] = make_double2(in ? y1 : 0.0, interior ? b1 : (in ? y2 - y1 : 0.0));
+    out[1] = make_double2(interior ? b2 : 0.0, interior ? b3 : 0.0);
+    cell->v[4] = in ? kCubicRound * big : 0.0;
+  }
+}
+
+__device__ __noinline__ float idiff_cubic_exact(const double* Y, int n, double x, float v) {
+  return static_cast<float>(static_cast<double>(v) + cubic_row(Y, n, x));
+}
+
+// One workgroup of 256 lanes owns a tile of (256 / LY) columns x LY P rows,
+// lane (cx, ly) the rows P ly ... P ly + P - 1 of its column, over all views
+// in order.  Windows are found for 128 views at a time and staged a.views at
+// a time, loaded into registers while the views before are interpolated (64
+// lanes a window, or 32 where it is short).  Every lane takes the views U at
+// a time.
+template <int INTERP, int LY, int P, int U>
+__global__ __launch_bounds__(kBlock) void bp_idiff_f64_kernel(IdiffArgs a) {
+  using Cell = IdiffCell<INTERP>;
+  extern __shared__ double2 s_dyn[];
+  Cell* const s_c = reinterpret_cast<Cell*>(s_dyn);  // [views][W]
+  __shared__ double s_v[kMeta][4];  // position of the tile's first pixel in the window, steps along x and y
+  __shared__ int2 s_win[kMeta];     // first interval, intervals
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  constexpr int kTx = kBlock / LY, kTy = LY * P;
+  const int ix0 = (tile / a.tilesY) * kTx, iy0 = (tile % a.tilesY) * kTy;
+  const int ix = ix0 + t / LY, iyb = iy0 + (t % LY) * P;
+  const int cx1 = min(ix0 + kTx - 1, a.nx - 1), cy1 = min(iy0 + kTy - 1, a.ny - 1);
+  const int W = a.W;
+  const double cx = t / LY, cy = (t % LY) * P;
+  const size_t pix = static_cast<size_t>(ix) * a.ny + iyb;
+  float v[P];
+#pragma unroll
+  for (int k = 0; k < P; k++) v[k] = ix < a.nx && iyb + k < a.ny ? a.image[pix + k] : 0.f;
+
+  // staging: `group` lanes take one window, 4 or 8 windows a pass; cells gl - 1
+  // + j0 of the window, of which the inner ones give intervals
+  const int group = a.half ? 32 : 64, gl = lane & (group - 1), inner = group - 3;
+  const int perPass = a.half ? 8 : 4, mine = a.half ? 2 * wave + (lane >> 5) : wave;
+  double raw[4];
+  int vb = 0, nb = 0;
+  auto load = [&](int view, int cell) {
+    return a.f[static_cast<size_t>(view) * a.nDet + min(max(cell, 0), a.nDet - 1)];
+  };
+  auto fetch = [&](int g) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int u = q * perPass + mine;
+      if (u < a.views && g + u < nb) raw[q] = load(vb + g + u, s_win[g + u].x + gl - 1);
+    }
+  };
+  auto place = [&](int g) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int u = q * perPass + mine;
+      if (q * perPass >= a.views) break;
+      const bool have = u < a.views && g + u < nb;
+      const int2 w = s_win[have ? g + u : g];
+      // (the loop's bound is the wave's: with 32 lanes a window, one round)
+      for (int j0 = 0; j0 < W; j0 += inner) {
+        const int j = j0 + gl - 1;
+        const double y1 = j0 == 0 ? raw[q] : load(vb + (have ? g + u : g), w.x + j);
+        const double y2 = lane_step<1>(y1), y3 = lane_step<1>(y2), y0 = lane_step<-1>(y1);
+        if (have && gl >= 1 && gl <= inner && j < w.y) idiff_coef<INTERP>(y0, y1, y2, y3, w.x + j, a.nDet, s_c + u * W + j);
+      }
+    }
+  };
+  // N views from view vv of those staged at v0 on
+  auto step = [&](int v0, int vv, auto count) {
+    constexpr int N = decltype(count)::value;
+    double pos[N][P], val[N][P], e[N][P];
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+      const double* c = s_v[v0 + vv + n];
+      pos[n][0] = fma(cx, c[1], fma(cy, c[2], c[0]));  // exact, and so are the steps
+#pragma unroll
+      for (int k = 1; k < P; k++) pos[n][k] = pos[n][k - 1] + c[2];
+#pragma unroll
+      for (int k = 0; k < P; k++) {
+        const double fr = __builtin_amdgcn_fract(pos[n][k]);
+        const int cell = min(max(static_cast<int>(pos[n][k]), 0), W - 1);  // (a pixel's: unchanged)
+        const Cell& q = s_c[(vv + n) * W + cell];
+        const double2* h = reinterpret_cast<const double2*>(q.v);
+        if constexpr (INTERP == INTERP_LINEAR) {
+          val[n][k] = h[0].x + fr * h[0].y;
+        } else {
+          val[n][k] = fma(fr, fma(fr, fma(fr, h[1].y, h[1].x), h[0].y), h[0].x);
+          e[n][k] = q.v[4];
+        }
+      }
+    }
+    if constexpr (INTERP == INTERP_LINEAR) {
+#pragma unroll
+      for (int n = 0; n < N; n++)
+#pragma unroll
+        for (int k = 0; k < P; k++) v[k] = static_cast<float>(static_cast<double>(v[k]) + val[n][k]);
+    } else {
+#pragma unroll
+      for (int n = 0; n < N; n++) {
+#pragma unroll
+        for (int k = 0; k < P; k++) {
+          const double vd = static_cast<double>(v[k]);
+          const float f0 = static_cast<float>(vd + (val[n][k] - e[n][k])), f1 = static_cast<float>(vd + (val[n][k] + e[n][k]));
+          const bool sure = (__float_as_uint(f0) == __float_as_uint(f1)) & (f0 == f0);
+          if (__builtin_expect(!sure, 0)) {
+            const int view = vb + v0 + vv + n;
+            v[k] = idiff_cubic_exact(a.f + static_cast<size_t>(view) * a.nDet, a.nDet, pos[n][k] + s_win[v0 + vv + n].x, v[k]);
+          } else {
+            v[k] = f0;
+          }
+        }
+      }
+    }
+  };
+
+  for (vb = 0; vb < a.nView; vb += kMeta) {
+    nb = min(kMeta, a.nView - vb);
+    if (t < nb) {
+      const ViewConstF64 c = a.vc[vb + t];
+      long long dx, dy, cs;
+      __builtin_memcpy(&dx, &c.a, 8);
+      __builtin_memcpy(&dy, &c.b, 8);
+      __builtin_memcpy(&cs, &c.c, 8);
+      const long long p0 = cs + ix0 * dx + iy0 * dy, p1 = cs + cx1 * dx + iy0 * dy;
+      const long long p2 = cs + ix0 * dx + cy1 * dy, p3 = cs + cx1 * dx + cy1 * dy;
+      const int lo = static_cast<int>(min(min(p0, p1), min(p2, p3)) >> 32);
+      const int hi = static_cast<int>(max(max(p0, p1), max(p2, p3)) >> 32);
+      s_win[t] = make_int2(lo, min(hi + 1 - lo, W));
+      s_v[t][0] = static_cast<double>(p0 - (static_cast<long long>(lo) << 32)) * 0x1p-32;
+      s_v[t][1] = static_cast<double>(dx) * 0x1p-32;
+      s_v[t][2] = static_cast<double>(dy) * 0x1p-32;
+    }
+    __syncthreads();  // the windows are there
+    fetch(0);
+    for (int v0 = 0; v0 < nb; v0 += a.views) {
+      const int nv = min(a.views, nb - v0);
+      place(v0);
+      __syncthreads();
+      if (v0 + a.views < nb) fetch(v0 + a.views);  // in flight during the interpolation below
+      int vv = 0;
+      for (; vv + U <= nv; vv += U) step(v0, vv, std::integral_constant<int, U>{});
+      for (; vv < nv; vv++) step(v0, vv, std::integral_constant<int, 1>{});
+      __syncthreads();  // every lane is done reading
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < P; k++)
+    if (ix < a.nx && iyb + k < a.ny) a.image[pix + k] = v[k];
+}
+
+// Cells of a window of tileX x tileY pixels, exactly: the positions of a
+// tile span at most the steps times its sides, and one cell for the ends.
+int idiff_window(const BpPlan& p, int tileX, int tileY) {
+  const double sx = (tileX - 1) * fabs(p.xInc) / p.detInc, sy = (tileY - 1) * fabs(p.yInc) / p.detInc;
+  const double w = ceil(sqrt(sx * sx + sy * sy) * (1 + 1e-9) + 1e-3) + 2;
+  return w < 4096 ? static_cast<int>(w) : 0;
+}
+
+size_t idiff_cell(const BpPlan& p) {
+  return p.interp == INTERP_CUBIC ? sizeof(IdiffCell<INTERP_CUBIC>) : sizeof(IdiffCell<INTERP_LINEAR>);
+}
+
 // Largest distance of a pixel from the origin.
 double pixel_radius(const BpPlan& p) {
   const double rx = fmax(fabs(p.xMin), fabs(p.xMax)), ry = fmax(fabs(p.yMin), fabs(p.yMax));
@@ -549,6 +764,50 @@ int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered,
   ctx->prof_begin();
   if (cubic) launch_fan_kind<INTERP_CUBIC>(p, deg, a, grid, lds, ctx->stream);
   else launch_fan_kind<INTERP_LINEAR>(p, deg, a, grid, lds, ctx->stream);
+  ctx->prof_end();
+  CTSIM_HIP(hipGetLastError());
+  return CTSIM_OK;
+}
+
+// The IntDiff kernel: positions below 2^20 cells (exact in FP64) and windows
+// that fit LDS four views at a time.
+bool bp_idiff_f64_ok(const BpPlan& p) {
+  if (p.kind != KIND_IDIFF || p.interp == INTERP_NEAREST || !(p.detInc > 0)) return false;
+  const double far = (fabs(p.xMin) + fabs(p.xMax) + fabs(p.yMin) + fabs(p.yMax)) / p.detInc + p.nDet;
+  const int W = idiff_window(p, 32, 32);
+  return far < 0x1p20 && W > 0 && 4 * W * idiff_cell(p) <= kFanLds;
+}
+
+int bp_idiff_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
+                        int nView, float* d_image) {
+  const bool cubic = p.interp == INTERP_CUBIC;
+  IdiffArgs a{};
+  a.nx = p.nx; a.ny = p.ny; a.nDet = p.nDet; a.nView = nView;
+  a.f = d_filtered; a.vc = d_vc; a.image = d_image;
+  // four rows per lane where that leaves four workgroups per CU, else one.
+  // Per slice with the FFT filter, one / four rows, linear: 256^2 47 / 96 us,
+  // 512^2 145 / 206, 1024^2 791 / 722; 2048^2 (convolution) 7.30 / 6.24 ms.
+  // Views at a time: 4 with one row, 2 (linear) or 1 (cubic, whose bounds take
+  // the registers) with four, each the fastest of 1, 2, 4 and 8.
+  const int P = static_cast<size_t>(p.nx) * p.ny >= static_cast<size_t>(4) * 4 * kBlock * ctx->numCUs ? 4 : 1;
+  const int side = P == 4 ? 32 : 16;
+  a.W = idiff_window(p, side, side);
+  a.tilesY = (p.ny + side - 1) / side;
+  const int grid = (p.nx + side - 1) / side * a.tilesY;
+  a.half = a.W <= 29;
+  for (a.views = 16; a.views > 4 && a.views * a.W * idiff_cell(p) > kFanLds; a.views /= 2) {
+  }
+  const size_t lds = a.views * a.W * idiff_cell(p);
+  const dim3 g(grid), b(kBlock);
+  const hipStream_t s = ctx->stream;
+  ctx->prof_begin();
+  if (cubic) {
+    if (P == 4) hipLaunchKernelGGL((bp_idiff_f64_kernel<INTERP_CUBIC, 8, 4, 1>), g, b, lds, s, a);
+    else hipLaunchKernelGGL((bp_idiff_f64_kernel<INTERP_CUBIC, 16, 1, 4>), g, b, lds, s, a);
+  } else {
+    if (P == 4) hipLaunchKernelGGL((bp_idiff_f64_kernel<INTERP_LINEAR, 8, 4, 2>), g, b, lds, s, a);
+    else hipLaunchKernelGGL((bp_idiff_f64_kernel<INTERP_LINEAR, 16, 1, 4>), g, b, lds, s, a);
+  }
   ctx->prof_end();
   CTSIM_HIP(hipGetLastError());
   return CTSIM_OK;

@@ -153,6 +153,10 @@ int bp_view_consts_mixed(ctsim_ctx* ctx, const BpPlan& p, const double* h_angles
 bool bp_fan_f64_ok(const BpPlan& p, double maxAngle);
 int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
                       int nView, float* d_image);
+// The same for the IntDiff FP64 kernel.
+bool bp_idiff_f64_ok(const BpPlan& p);
+int bp_idiff_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
+                        int nView, float* d_image);
 // True when the mixed precision of this plan runs the tiled coefficient
 // kernel (not the FP64 index path) and one view's staging fits LDS.
 bool bp_mixed_tiled(const BpPlan& p);

@@ -14,8 +14,9 @@ from ctsim_amd import workloads as W
 pytestmark = pytest.mark.gpu
 
 
-def _scan(O, geom, nDet, nView):
-    return O.Phantom(None, W.mixed_elements(31)), O.ScanSpec(geom, nDet, nView, 0, 1, 2 * np.pi)
+def _scan(O, geom, nDet, nView, scanRatio=1.0):
+    return (O.Phantom(None, W.mixed_elements(31)),
+            O.ScanSpec(geom, nDet, nView, 0, 1, 2 * np.pi, 2.0, 2.0, 1.0, scanRatio))
 
 
 def _plan(ctx, geom, nDet, nView, nx, ny, interp, info):
@@ -24,30 +25,31 @@ def _plan(ctx, geom, nDet, nView, nx, ny, interp, info):
                                    info["focalLength"], info["sourceDetectorLength"], "idiff", interp, nx, ny)
 
 
-def _info(geom, nDet, nView):
+def _info(geom, nDet, nView, scanRatio=1.0):
     import ctsim_amd
     return ctsim_amd.Scanner(ctsim_amd.Phantom(None, W.mixed_elements(31)), geom, nDet, nView, 0, 1,
-                             2 * np.pi).info
+                             2 * np.pi, 2.0, 2.0, 1.0, scanRatio).info
 
 
-# image, detectors, views: degree 14 (24, 40 and 64 pixels across), 8 (130, 200), 5 (320); the last row's
+# image, detectors, views, scan ratio (0.5: the detector ends inside the image): degree 14 (24, 40 and 64 pixels across), 8 (130, 200), 5 (320); the last row's
 # windows are too long to stage, so the general kernel runs
-SHAPES = [(16, 16, 65, 1), (17, 33, 66, 7), (24, 1, 65, 8), (40, 64, 97, 9), (130, 95, 200, 129), (200, 33, 367, 12),
-          (320, 31, 500, 131), (33, 17, 1200, 5), (20, 20, 3000, 4)]
+SHAPES = [(16, 16, 65, 1, 1.0), (17, 33, 66, 7, 1.0), (24, 1, 65, 8, 1.0), (40, 64, 97, 9, 1.0),
+          (130, 95, 200, 129, 1.0), (200, 33, 367, 12, 1.0), (320, 31, 500, 131, 1.0), (64, 50, 97, 33, 0.5),
+          (33, 17, 1200, 5, 1.0), (20, 20, 3000, 4, 1.0)]
 
 
 @pytest.mark.parametrize("interp", ["linear", "cubic"])
 @pytest.mark.parametrize("geom", ["equiangular", "equilinear"])
-@pytest.mark.parametrize("nx,ny,nDet,nView", SHAPES)
-def test_noise_rows_match_oracle(gpu_ctx, oracle_lib, geom, interp, nx, ny, nDet, nView):
+@pytest.mark.parametrize("nx,ny,nDet,nView,scanRatio", SHAPES)
+def test_noise_rows_match_oracle(gpu_ctx, oracle_lib, geom, interp, nx, ny, nDet, nView, scanRatio):
     import torch
     import ctsim_amd
     print(f"case fan f64 {geom} {interp} {nx}x{ny} {nDet}x{nView}", flush=True)
-    phm, scan = _scan(oracle_lib, geom, nDet, nView)
+    phm, scan = _scan(oracle_lib, geom, nDet, nView, scanRatio)
     rows = np.random.default_rng(nx + nView).standard_normal((nView, nDet))
     angles = np.arange(nView) * (2 * np.pi / nView)
     want = oracle_lib.backproject("oracle", phm, scan, "idiff", interp, nx, ny, rows, angles)
-    info = _info(geom, nDet, nView)
+    info = _info(geom, nDet, nView, scanRatio)
     b = _plan(gpu_ctx, geom, nDet, nView, nx, ny, interp, info)
     img = torch.zeros((nx, ny), dtype=torch.float32, device="cuda")
     b.backproject(torch.from_numpy(rows).cuda(), angles, img, ctsim_amd.PREC_F64)
