@@ -26,72 +26,85 @@ constexpr int kLanes = 64;        // views per wave
 constexpr int kWaves = 4;         // waves per block
 constexpr int kOutPerWave = 8;    // outputs per wave (independent sums)
 constexpr int kJChunk = 64;       // inputs staged per step
-constexpr int kConvOut = 16;      // exact convolution: outputs per lane (independent sums)
+constexpr int kTapPad = 4 * 8 + 8;  // zeros after the exact convolution's taps: a block's outputs beyond n
 constexpr int kKChunk = 32;       // spectrum entries staged per step (inverse DFT)
 
 // ---------------------------------------------------- exact convolution
 // out[v][i] = dx * sum_{j=0}^{n-1} x[v][j] * h[i - j + n - 1]  (procsignal.cpp:659-673)
-template <class TO>
+//
+// Lanes are views; a wave owns O consecutive outputs, a block 4 O.  Every
+// step's taps are the same for the whole wave, so they come through scalar
+// loads from the plan's table (kTapPad zeros after the last tap, which only
+// outputs beyond n read); the projections of 64 views, weighted in FP64 as
+// the reference does, pass through LDS, loaded along the detector (one row a
+// wave and step) while the chunk before is summed.
+//
+// What bounds it: FP64 VALU issue; the products and sums are two instructions
+// per step and output (they may not be fused), and nothing else is in the
+// loop.  2880 rows of 2048 detectors: 1.66 ms with the taps in LDS and the
+// rows loaded across the views, 0.72 ms here; 320 rows of 367, 30 blocks of
+// 64 x 64 sums before: 75 us and 17.
+template <int O>
 __global__ __launch_bounds__(kLanes * kWaves) void conv_seq_kernel(
     const float* __restrict__ in, const double* __restrict__ w, const double* __restrict__ h,
-    TO* __restrict__ out, int nView, int n, double dx, int outStride) {
-  __shared__ double s_x[kJChunk][kLanes];
-  extern __shared__ double s_h[];  // the block's taps: h[ib + k], k < n + kWaves * kConvOut - 1
-  const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
-  const int v = blockIdx.y * kLanes + lane;
-  const int ib = blockIdx.x * kWaves * kConvOut, i0 = ib + wave * kConvOut;
-  // output i of the block at input j takes tap i - j + n - 1, in [ib, ib + n - 1 + kWaves kConvOut)
-  const int nTap = n + kWaves * kConvOut - 1;
-  for (int k = threadIdx.x; k < nTap; k += blockDim.x) s_h[k] = h[min(ib + k, 2 * n - 2)];
-  double acc[kConvOut];
+    double* __restrict__ out, int nView, int n, double dx, int outStride) {
+  __shared__ double s_x[kJChunk][kLanes + 1];
+  const int lane = threadIdx.x & (kLanes - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
+  const int vb = blockIdx.y * kLanes, v = vb + lane;
+  const int i0 = (blockIdx.x * kWaves + wave) * O;
+  constexpr int kRows = kLanes / kWaves;  // rows a wave loads: wave, wave + 4, ...
+  float raw[kRows];
+  auto fetch = [&](int j0) {
+    const int j = j0 + lane;
 #pragma unroll
-  for (int o = 0; o < kConvOut; o++) acc[o] = 0.0;
+    for (int r = 0; r < kRows; r++) {
+      const int vv = vb + wave + r * kWaves;
+      raw[r] = j < n && vv < nView ? in[static_cast<size_t>(vv) * n + j] : 0.f;
+    }
+  };
+  double acc[O];
+#pragma unroll
+  for (int o = 0; o < O; o++) acc[o] = 0.0;
+  fetch(0);
   for (int j0 = 0; j0 < n; j0 += kJChunk) {
-    __syncthreads();
-    for (int k = threadIdx.x; k < kJChunk * kLanes; k += blockDim.x) {
-      const int jj = k / kLanes, l = k % kLanes;
-      const int j = j0 + jj, vv = blockIdx.y * kLanes + l;
-      double xv = 0.0;
-      if (j < n && vv < nView) {
-        xv = static_cast<double>(in[static_cast<size_t>(vv) * n + j]);
-        if (w) xv *= w[j];
+    __syncthreads();  // the last chunk's readers are done
+    {
+      const double wj = w && j0 + lane < n ? w[j0 + lane] : 1.0;
+#pragma unroll
+      for (int r = 0; r < kRows; r++) {
+        double xv = static_cast<double>(raw[r]);
+        if (w) xv *= wj;
+        s_x[lane][wave + r * kWaves] = xv;
       }
-      s_x[jj][l] = xv;
     }
     __syncthreads();
+    if (j0 + kJChunk < n) fetch(j0 + kJChunk);  // in flight during the sums below
     const int jn = min(kJChunk, n - j0);
     int jj = 0;
     // 8 steps at a time: output o at step j + u takes tap i0 + o - j - u +
-    // n - 1, so one window of kConvOut + 7 taps serves the block (T[7 + o -
-    // u]); every sum still adds its products in input order
+    // n - 1, so one window of O + 7 taps serves them (T[7 + o - u]); every
+    // sum adds its products in input order
     for (; jj + 8 <= jn; jj += 8) {
-      const int base = i0 - (j0 + jj) + n - 1 - 7 - ib;  // local tap index of T[0]
-      double T[kConvOut + 7];
-#pragma unroll
-      for (int m = 0; m < kConvOut + 7; m++) T[m] = s_h[max(base + m, 0)];
+      const double* T = h + (i0 - (j0 + jj) + n - 1 - 7);
 #pragma unroll
       for (int u = 0; u < 8; u++) {
         const double xv = s_x[jj + u][lane];
 #pragma unroll
-        for (int o = 0; o < kConvOut; o++)
-          if (i0 + o < n) acc[o] += xv * T[7 + o - u];
+        for (int o = 0; o < O; o++) acc[o] += xv * T[7 + o - u];
       }
     }
     for (; jj < jn; jj++) {
       const double xv = s_x[jj][lane];
-      const int j = j0 + jj;
+      const double* T = h + (i0 - (j0 + jj) + n - 1);
 #pragma unroll
-      for (int o = 0; o < kConvOut; o++) {
-        const int i = i0 + o;
-        if (i < n) acc[o] += xv * s_h[i - j + n - 1 - ib];
-      }
+      for (int o = 0; o < O; o++) acc[o] += xv * T[o];
     }
   }
   if (v < nView) {
 #pragma unroll
-    for (int o = 0; o < kConvOut; o++) {
+    for (int o = 0; o < O; o++) {
       const int i = i0 + o;
-      if (i < n) out[static_cast<size_t>(v) * outStride + i] = static_cast<TO>(acc[o] * dx);
+      if (i < n) out[static_cast<size_t>(v) * outStride + i] = acc[o] * dx;
     }
   }
 }
@@ -548,9 +561,10 @@ int launch_fft(ctsim_ctx* ctx, const FilterPlan& p, const float* d_in, int nView
 }  // namespace
 
 int filter_upload(FilterPlan& p) {
-  CTSIM_CHECK(p.d_filter.reserve(p.filter.size() * sizeof(double)));
-  CTSIM_HIP(hipMemcpy(p.d_filter.ptr, p.filter.data(), p.filter.size() * sizeof(double),
-                      hipMemcpyHostToDevice));
+  std::vector<double> taps(p.filter);
+  taps.resize(p.filter.size() + kTapPad, 0.0);
+  CTSIM_CHECK(p.d_filter.reserve(taps.size() * sizeof(double)));
+  CTSIM_HIP(hipMemcpy(p.d_filter.ptr, taps.data(), taps.size() * sizeof(double), hipMemcpyHostToDevice));
   if (!p.preweight.empty()) {
     CTSIM_CHECK(p.d_weight.reserve(p.preweight.size() * sizeof(double)));
     CTSIM_HIP(hipMemcpy(p.d_weight.ptr, p.preweight.data(), p.preweight.size() * sizeof(double),
@@ -739,16 +753,19 @@ int filter_launch(ctsim_ctx* ctx, FilterPlan& p, int precision, const float* d_i
     return CTSIM_OK;
   }
   if (p.method == METHOD_CONVOLUTION) {
-    const dim3 grid((p.n + kWaves * kConvOut - 1) / (kWaves * kConvOut), (nView + kLanes - 1) / kLanes);
-    const size_t lds = static_cast<size_t>(p.n + kWaves * kConvOut - 1) * sizeof(double);
-    if (lds + sizeof(double) * kJChunk * kLanes > 64 * 1024)
-      return fail(CTSIM_ERR_UNSUPPORTED, "convolution filter: kernel too long for LDS");
-    if (f64)
-      hipLaunchKernelGGL((conv_seq_kernel<double>), grid, dim3(kLanes * kWaves), lds, s, d_in, w,
-                         p.d_filter.as<double>(), static_cast<double*>(d_out), nView, p.n, p.inc, outStride);
-    else
-      hipLaunchKernelGGL((conv_seq_kernel<float>), grid, dim3(kLanes * kWaves), lds, s, d_in, w,
-                         p.d_filter.as<double>(), static_cast<float*>(d_out), nView, p.n, p.inc, outStride);
+    if (p.n > 4033) return fail(CTSIM_ERR_UNSUPPORTED, "convolution filter: kernel too long for LDS");
+    // 8 outputs per wave where that gives a block to every CU, else 4 or 2 (a
+    // whole slice, 2 / 4 / 8 outputs: 320 x 367 62 / 65 / 70 us, 731 x 701
+    // 447 / 421 / 418, 1440 x 1024 500 / 459 / 435; 16 gain nothing at 2880 x 2048)
+    auto blocks = [&](int O) { return ((p.n + kWaves * O - 1) / (kWaves * O)) * ((nView + kLanes - 1) / kLanes); };
+    auto go = [&](auto kern, int O) {
+      hipLaunchKernelGGL(kern, dim3((p.n + kWaves * O - 1) / (kWaves * O), (nView + kLanes - 1) / kLanes),
+                         dim3(kLanes * kWaves), 0, s, d_in, w, p.d_filter.as<double>(), static_cast<double*>(d_out),
+                         nView, p.n, p.inc, outStride);
+    };
+    if (blocks(8) >= ctx->numCUs) go(conv_seq_kernel<8>, 8);
+    else if (blocks(4) >= ctx->numCUs) go(conv_seq_kernel<4>, 4);
+    else go(conv_seq_kernel<2>, 2);
     CTSIM_HIP(hipGetLastError());
     return CTSIM_OK;
   }
