@@ -644,9 +644,22 @@ int bp_upload_tables(BpPlan& p) {
   return CTSIM_OK;
 }
 
+namespace {
+
+int fill_image(ctsim_ctx* ctx, const BpPlan& p, float* d_image) {
+  const size_t npix = static_cast<size_t>(p.nx) * p.ny;
+  int g = static_cast<int>((npix + 255) / 256);
+  if (g > 4096) g = 4096;
+  hipLaunchKernelGGL(bp_fill_kernel, dim3(g), dim3(256), 0, ctx->stream, d_image, npix, 0.f);
+  CTSIM_HIP(hipGetLastError());
+  return CTSIM_OK;
+}
+
+}  // namespace
+
 int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filtered,
-              const double* h_angles, int nView, float* d_image) {
-  if (nView <= 0) return CTSIM_OK;
+              const double* h_angles, int nView, float* d_image, bool fresh) {
+  if (nView <= 0) return fresh ? fill_image(ctx, p, d_image) : CTSIM_OK;
   const hipStream_t s = ctx->stream;
   BpArgs a{};
   a.nx = p.nx; a.ny = p.ny; a.nDet = p.nDet; a.iDetCenter = p.iDetCenter; a.nView = nView;
@@ -687,16 +700,17 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
         &a.vc));
     if (!inF32 && bp_fan_f64_ok(p, p.cachedMaxAngle))
       return bp_fan_f64_launch(ctx, p, static_cast<const double*>(d_filtered),
-                               static_cast<const ViewConstF64*>(a.vc), nView, d_image);
+                               static_cast<const ViewConstF64*>(a.vc), nView, d_image, fresh);
     if (!inF32 && bp_idiff_f64_ok(p))
       return bp_idiff_f64_launch(ctx, p, static_cast<const double*>(d_filtered),
-                                 static_cast<const ViewConstF64*>(a.vc), nView, d_image);
+                                 static_cast<const ViewConstF64*>(a.vc), nView, d_image, fresh);
+    if (fresh) CTSIM_CHECK(fill_image(ctx, p, d_image));
     if (p.kind == KIND_DIFF) {
       const int g = (p.nx + 63) / 64;
       if (inF32) launch_diff<float>(p.interp, a, g, s);
       else launch_diff<double>(p.interp, a, g, s);
       CTSIM_HIP(hipGetLastError());
-      return CTSIM_OK;
+      return fresh ? bp_launch_post(ctx, p, d_image) : CTSIM_OK;
     }
     a.W = p.windowF64;
     const int Wv = a.W > 0 ? a.W : p.nDet + 8;
@@ -712,13 +726,15 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
     else launch_f64_interp<double>(p.interp, p.kind, a, grid, lds, s);
     ctx->prof_end();
     CTSIM_HIP(hipGetLastError());
-    return CTSIM_OK;
+    return fresh ? bp_launch_post(ctx, p, d_image) : CTSIM_OK;
   }
+  if (fresh) CTSIM_CHECK(fill_image(ctx, p, d_image));
 
   const ViewConstF32* vc32 = nullptr;
   CTSIM_CHECK(bp_view_consts_mixed(ctx, p, h_angles, nView, &vc32));
-  return bp_launch_mixed(ctx, p, p.mixed, static_cast<const float*>(d_filtered), vc32, nView,
-                         d_image);
+  CTSIM_CHECK(bp_launch_mixed(ctx, p, p.mixed, static_cast<const float*>(d_filtered), vc32, nView,
+                              d_image));
+  return fresh ? bp_launch_post(ctx, p, d_image) : CTSIM_OK;
 }
 
 // The symmetric kernel applies to a square centred grid, views with a
@@ -1108,22 +1124,17 @@ int ctsim_fbp_slice(ctsim_ctx* ctx, ctsim_procsignal* ps, const ctsim_backprojec
     return fail(CTSIM_ERR_INVALID, "ctsim_fbp_slice: filter and backprojector detector counts differ");
   CTSIM_CHECK(ctx->activate());
   const hipStream_t s = ctx->stream;
-  const size_t npix = static_cast<size_t>(p.nx) * p.ny;
   const bool mixed = precision == CTSIM_PREC_MIXED;
   if (!mixed || !bp_mixed_tiled(p) || p.interpFactor != 1 || nView == 0) {
     // The separate steps (pjrec: zeroed image, filterSignal, BackprojectView
     // per view, PostProcessing).
-    int g = static_cast<int>((npix + 255) / 256);
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL(bp_fill_kernel, dim3(g), dim3(256), 0, s, d_image, npix, 0.f);
-    CTSIM_HIP(hipGetLastError());
-    if (nView == 0) return CTSIM_OK;
-    const int stride = f.n * f.preinterp;
-    CTSIM_CHECK(ctx->scratch3.reserve(static_cast<size_t>(nView) * stride *
-                                      (mixed ? sizeof(float) : sizeof(double))));
-    CTSIM_CHECK(filter_launch(ctx, f, precision, d_sino, nView, ctx->scratch3.ptr, stride));
-    CTSIM_CHECK(bp_launch(ctx, p, precision, ctx->scratch3.ptr, h_angles, nView, d_image));
-    return bp_launch_post(ctx, p, d_image);
+    if (nView > 0) {
+      const int stride = f.n * f.preinterp;
+      CTSIM_CHECK(ctx->scratch3.reserve(static_cast<size_t>(nView) * stride *
+                                        (mixed ? sizeof(float) : sizeof(double))));
+      CTSIM_CHECK(filter_launch(ctx, f, precision, d_sino, nView, ctx->scratch3.ptr, stride));
+    }
+    return bp_launch(ctx, p, precision, ctx->scratch3.ptr, h_angles, nView, d_image, true);
   }
   // Mixed and tiled: the filter writes interval coefficients (FFT methods
   // straight from LDS; convolution through float rows), then the tiled

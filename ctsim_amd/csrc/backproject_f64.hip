@@ -70,6 +70,8 @@ struct FanF64Args {
   const double* f;
   const ViewConstF64* vc;
   float* image;
+  double endScale;            // fresh: factor applied to the finished sums
+  int fresh;                  // sums start at zero instead of the image
   double posScale;            // equilinear: sdl / detInc
   double atan[kMaxDeg + 1];   // equiangular: series of atan(t)/t in t^2, over detInc
   FanBounds b;
@@ -218,6 +220,16 @@ __device__ __forceinline__ void fan_pos(const FanF64Args& a, double rc, double f
   }
 }
 
+// The kernel's arguments where they are used once in a long while: read again
+// each time, instead of being held (and spilled) in scalar registers that the
+// inner loop needs.
+typedef const __attribute__((address_space(4))) FanF64Args* FanArgsPtr;
+__device__ __forceinline__ FanArgsPtr cold_args() {
+  FanArgsPtr p = (FanArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // One workgroup of 256 lanes owns a tile of 16 x 16 pixels, one per lane
 // (lanes along iy), over all views (the float32 sums are in view order).
 // Constants and windows are found for 128 views at a time, one view per
@@ -250,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void bp_fan_f64_kernel(FanF64Args a) {
   const int W = a.W;
   const double x = a.xs[min(ix, a.nx - 1)], y = a.ys[min(iy, a.ny - 1)];
   const size_t pix = static_cast<size_t>(ix) * a.ny + iy;
-  float v = active ? a.image[pix] : 0.f;
+  float v = active && !a.fresh ? a.image[pix] : 0.f;
 
   // the cells of this wave's two views of the eight at view g (zero outside
   // the detector, and for views beyond nb)
@@ -295,20 +307,21 @@ __global__ __launch_bounds__(kBlock) void bp_fan_f64_kernel(FanF64Args a) {
   for (vb = 0; vb < a.nView; vb += kMeta) {
     nb = min(kMeta, a.nView - vb);
     if (t < nb) {
-      const ViewConstF64 c = a.vc[vb + t];
-      const double xa = a.xs[ix0], xb = a.xs[cx1], ya = a.ys[iy0], yb = a.ys[cy1];
-      double ct = c.a, st = c.b, Fs = 0.0, Fc = a.F, base = a.center;
+      const FanArgsPtr ca = cold_args();
+      const ViewConstF64 c = ca->vc[vb + t];
+      const double xa = ca->xs[ix0], xb = ca->xs[cx1], ya = ca->ys[iy0], yb = ca->ys[cy1];
+      double ct = c.a, st = c.b, Fs = 0.0, Fc = ca->F, base = ca->center;
       const double xm = 0.5 * (xa + xb), ym = 0.5 * (ya + yb);
       if constexpr (KIND == KIND_EQUIANGULAR) {
-        const double a0 = crm_atan(fma(xm, ct, ym * st) / (a.F + fma(xm, st, -(ym * ct))));
-        double sa, ca;
-        crm_sincos(a0, &sa, &ca);
+        const double a0 = crm_atan(fma(xm, ct, ym * st) / (ca->F + fma(xm, st, -(ym * ct))));
+        double sa, co;
+        crm_sincos(a0, &sa, &co);
         const double ct0 = ct, st0 = st;
-        ct = fma(ct0, ca, -(st0 * sa));
-        st = fma(st0, ca, ct0 * sa);
-        Fs = -a.F * sa;
-        Fc = a.F * ca;
-        base += a0 / a.detInc;
+        ct = fma(ct0, co, -(st0 * sa));
+        st = fma(st0, co, ct0 * sa);
+        Fs = -ca->F * sa;
+        Fc = ca->F * co;
+        base += a0 / ca->detInc;
       }
       double pmin = 1e300, pmax = -1e300;
 #pragma unroll
@@ -323,13 +336,13 @@ __global__ __launch_bounds__(kBlock) void bp_fan_f64_kernel(FanF64Args a) {
       const double dA = ldexp(0x1p-53, __builtin_amdgcn_frexp_exp(fabs(c.theta) + 3.15) - 1);
       const double flm = fma(-ym, ct, fma(xm, st, Fc)), rcm = fma(ym, st, fma(xm, ct, Fs));
       const double L = sqrt(fma(flm, flm, rcm * rcm));
-      const double perp = fma(a.b.rA, dA, a.b.dPerp);
+      const double perp = fma(ca->b.rA, dA, ca->b.dPerp);
       if constexpr (KIND == KIND_EQUIANGULAR) {
-        s_v[t][5] = fma(a.b.kPos, perp / (L - a.b.radius) + a.b.extra, a.b.posC);
+        s_v[t][5] = fma(ca->b.kPos, perp / (L - ca->b.radius) + ca->b.extra, ca->b.posC);
       } else {
-        const double fl = flm - a.b.radius;
-        s_v[t][5] = fma(a.b.kPos, perp * (L + a.b.radius) / (fl * fl),
-                        fma(a.b.posR, fmax(fabs(pmin - base), fabs(pmax - base)), a.b.posC));
+        const double fl = flm - ca->b.radius;
+        s_v[t][5] = fma(ca->b.kPos, perp * (L + ca->b.radius) / (fl * fl),
+                        fma(ca->b.posR, fmax(fabs(pmin - base), fabs(pmax - base)), ca->b.posC));
       }
       // positions that are no numbers stage anything: every pixel then fails its tests
       if (!(pmin > -1e9 && pmin < 1e9)) pmin = 0;
@@ -382,10 +395,13 @@ __global__ __launch_bounds__(kBlock) void bp_fan_f64_kernel(FanF64Args a) {
         for (int n = 0; n < N; n++) {
           const int view = vb + v0 + vv + n;
           const float f0 = static_cast<float>(fma(w[n], lo[n], static_cast<double>(v)));
-          if (sure(n, f0)) v = f0;
-          else
-            v = fan_exact<KIND, INTERP>(a.r[pix], a.phi[pix], a.vc[view].theta, a.F, a.sdl, a.detInc, a.center, a.nDet,
-                                        a.f + static_cast<size_t>(view) * a.nDet, v);
+          if (sure(n, f0)) {
+            v = f0;
+          } else {
+            const FanArgsPtr ca = cold_args();
+            v = fan_exact<KIND, INTERP>(ca->r[pix], ca->phi[pix], ca->vc[view].theta, ca->F, ca->sdl, ca->detInc,
+                                        ca->center, ca->nDet, ca->f + static_cast<size_t>(view) * ca->nDet, v);
+          }
         }
       }
     };
@@ -402,7 +418,10 @@ __global__ __launch_bounds__(kBlock) void bp_fan_f64_kernel(FanF64Args a) {
       __syncthreads();  // every lane is done reading
     }
   }
-  if (active) a.image[pix] = v;
+  if (active) {
+    const FanArgsPtr ca = cold_args();
+    ca->image[pix] = ca->fresh ? static_cast<float>(static_cast<double>(v) * ca->endScale) : v;
+  }
 }
 
 template <int KIND, int INTERP, int DEG>
@@ -440,6 +459,8 @@ void launch_fan_kind(const BpPlan& p, int deg, const FanF64Args& a, int grid, si
 struct IdiffArgs {
   int nx, ny, nDet, nView;
   int tilesY, W, views, half;  // views: staged at a time; half: 32 lanes stage a window
+  int fresh;                   // as in FanF64Args
+  double endScale;
   const double* f;
   const ViewConstF64* vc;
   float* image;
@@ -502,7 +523,7 @@ __global__ __launch_bounds__(kBlock) void bp_idiff_f64_kernel(IdiffArgs a) {
   const size_t pix = static_cast<size_t>(ix) * a.ny + iyb;
   float v[P];
 #pragma unroll
-  for (int k = 0; k < P; k++) v[k] = ix < a.nx && iyb + k < a.ny ? a.image[pix + k] : 0.f;
+  for (int k = 0; k < P; k++) v[k] = !a.fresh && ix < a.nx && iyb + k < a.ny ? a.image[pix + k] : 0.f;
 
   // staging: `group` lanes take one window, 4 or 8 windows a pass; cells gl - 1
   // + j0 of the window, of which the inner ones give intervals
@@ -616,7 +637,8 @@ __global__ __launch_bounds__(kBlock) void bp_idiff_f64_kernel(IdiffArgs a) {
   }
 #pragma unroll
   for (int k = 0; k < P; k++)
-    if (ix < a.nx && iyb + k < a.ny) a.image[pix + k] = v[k];
+    if (ix < a.nx && iyb + k < a.ny)
+      a.image[pix + k] = a.fresh ? static_cast<float>(static_cast<double>(v[k]) * a.endScale) : v[k];
 }
 
 // Cells of a window of tileX x tileY pixels, exactly: the positions of a
@@ -742,7 +764,7 @@ bool bp_fan_f64_ok(const BpPlan& p, double maxAngle) {
 }
 
 int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
-                      int nView, float* d_image) {
+                      int nView, float* d_image, bool fresh) {
   const bool cubic = p.interp == INTERP_CUBIC, equi = p.kind == KIND_EQUIANGULAR;
   FanF64Args a{};
   a.nx = p.nx; a.ny = p.ny; a.nDet = p.nDet; a.center = p.iDetCenter; a.nView = nView;
@@ -757,6 +779,7 @@ int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered,
   a.xs = a.r + 2 * n;
   a.ys = a.xs + p.nx;
   a.f = d_filtered; a.vc = d_vc; a.image = d_image;
+  a.fresh = fresh; a.endScale = p.rotScale;
   const int deg = equi ? atan_degree(p) : 0;
   for (int k = 0; k <= deg; k++) a.atan[k] = (k & 1 ? -1.0 : 1.0) / ((2 * k + 1) * p.detInc);
   a.posScale = p.sdl / p.detInc;
@@ -779,11 +802,12 @@ bool bp_idiff_f64_ok(const BpPlan& p) {
 }
 
 int bp_idiff_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
-                        int nView, float* d_image) {
+                        int nView, float* d_image, bool fresh) {
   const bool cubic = p.interp == INTERP_CUBIC;
   IdiffArgs a{};
   a.nx = p.nx; a.ny = p.ny; a.nDet = p.nDet; a.nView = nView;
   a.f = d_filtered; a.vc = d_vc; a.image = d_image;
+  a.fresh = fresh; a.endScale = p.rotScale;
   // four rows per lane where that leaves four workgroups per CU, else one.
   // Per slice with the FFT filter, one / four rows, linear: 256^2 47 / 96 us,
   // 512^2 145 / 206, 1024^2 791 / 722; 2048^2 (convolution) 7.30 / 6.24 ms.

@@ -130,8 +130,11 @@ MixedShape bp_default_shape(const BpPlan& p, int numCUs);
 
 // Device side (backproject.hip).
 int bp_upload_tables(BpPlan& p);
+// Adds the views to the image; fresh: to an image of zeros, and scales the sum
+// as PostProcessing does (the FP64 fan-beam and IntDiff kernels without a pass
+// of their own for either).
 int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filtered,
-              const double* h_angles, int nView, float* d_image);
+              const double* h_angles, int nView, float* d_image, bool fresh = false);
 int bp_launch_post(ctsim_ctx* ctx, const BpPlan& p, float* d_image);
 int bp_launch_mixed(ctsim_ctx* ctx, const BpPlan& p, const MixedShape& m, const float* d_filtered,
                     const ViewConstF32* d_vc, int nView, float* d_image);
@@ -152,11 +155,11 @@ int bp_view_consts_mixed(ctsim_ctx* ctx, const BpPlan& p, const double* h_angles
 // angles up to maxAngle in size, and its launch over nView filtered rows.
 bool bp_fan_f64_ok(const BpPlan& p, double maxAngle);
 int bp_fan_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
-                      int nView, float* d_image);
+                      int nView, float* d_image, bool fresh);
 // The same for the IntDiff FP64 kernel.
 bool bp_idiff_f64_ok(const BpPlan& p);
 int bp_idiff_f64_launch(ctsim_ctx* ctx, const BpPlan& p, const double* d_filtered, const ViewConstF64* d_vc,
-                        int nView, float* d_image);
+                        int nView, float* d_image, bool fresh);
 // True when the mixed precision of this plan runs the tiled coefficient
 // kernel (not the FP64 index path) and one view's staging fits LDS.
 bool bp_mixed_tiled(const BpPlan& p);
