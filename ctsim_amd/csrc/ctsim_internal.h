@@ -93,6 +93,7 @@ struct ctsim_ctx {
   ctsim::DevBuf helixGam, helixErr;
   int helixGeom = -1, helixNDet = 0;
   double helixDetInc = 0, helixSdl = 0;
+  ctsim::DevBuf rasterTab;    // coordinates and sums of the rasteriser's last call
   int numCUs = 256;
   int activate() const;       // hipSetDevice(device)
   // Kernel timing: while enabled, the main backprojection kernel of each
