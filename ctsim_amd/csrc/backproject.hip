@@ -732,9 +732,13 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
 
   const ViewConstF32* vc32 = nullptr;
   CTSIM_CHECK(bp_view_consts_mixed(ctx, p, h_angles, nView, &vc32));
-  CTSIM_CHECK(bp_launch_mixed(ctx, p, p.mixed, static_cast<const float*>(d_filtered), vc32, nView,
-                              d_image));
+  CTSIM_CHECK(bp_launch_mixed(ctx, p, bp_mixed_shape(p, p.cachedSym, nView), static_cast<const float*>(d_filtered),
+                              vc32, nView, d_image));
   return fresh ? bp_launch_post(ctx, p, d_image) : CTSIM_OK;
+}
+
+MixedShape bp_mixed_shape(const BpPlan& p, const SymViews& sv, int nView) {
+  return p.mixedTuned ? p.mixed : bp_auto_shape(p, sv, nView);
 }
 
 // The symmetric kernel applies to a square centred grid, views with a
@@ -915,6 +919,28 @@ int bp_mixed_tiles(ctsim_ctx* ctx, const BpPlan& p, const MixedShape& m, const v
   }
   CTSIM_HIP(hipGetLastError());
   return CTSIM_OK;
+}
+
+namespace {
+size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
+}  // namespace
+
+SliceScratch fbp_slice_scratch(const FilterPlan& f, const BpPlan& p, const MixedShape& m, int nView) {
+  const bool coefFilter = filter_can_coef(f);
+  const int split = m.split < 1 ? 1 : (m.split > nView ? nView : m.split);
+  SliceScratch s;
+  s.vc = align256(sizeof(ViewConstF32) * nView);
+  s.coef = align256(static_cast<size_t>(nView) * p.nDet * (p.interp == INTERP_CUBIC ? sizeof(float4) : sizeof(float2)));
+  s.rows = coefFilter ? 0 : align256(static_cast<size_t>(nView) * f.n * sizeof(float));
+  s.work = coefFilter ? 0 : align256(filter_work_bytes(f, CTSIM_PREC_MIXED, nView));
+  s.partial = split > 1 ? align256(static_cast<size_t>(split) * p.nx * p.ny * sizeof(float)) : 0;
+  return s;
+}
+
+MixedShape fbp_slice_shape(const FilterPlan& f, const BpPlan& p, const SymViews& sv, int nView) {
+  const MixedShape m = bp_mixed_shape(p, sv, nView);
+  if (p.mixedTuned || fbp_slice_scratch(f, p, m, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES) return m;
+  return fbp_slice_scratch(f, p, p.mixed, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES ? p.mixed : m;
 }
 
 // Per-view FP32 constants of a mixed launch on the device (cached by angles).
@@ -1107,6 +1133,7 @@ int ctsim_backprojector_set_shape(ctsim_backprojector* bp, const int* shape6) {
   if (static_cast<size_t>(chunk) * Wv * (bp->plan.interp == INTERP_CUBIC ? 16 : 8) > kMixedLdsMax)
     return fail(CTSIM_ERR_INVALID, "ctsim_backprojector_set_shape: staging exceeds 64 KB of LDS");
   bp->plan.mixed = m;
+  bp->plan.mixedTuned = true;
   return CTSIM_OK;
 }
 
@@ -1152,7 +1179,8 @@ int ctsim_fbp_slice(ctsim_ctx* ctx, ctsim_procsignal* ps, const ctsim_backprojec
   }
   const ViewConstF32* vc = nullptr;
   CTSIM_CHECK(bp_view_consts_mixed(ctx, p, h_angles, nView, &vc));
-  return bp_mixed_tiles(ctx, p, p.mixed, ctx->scratch2.ptr, vc, nView, d_image, p.rotScale, true);
+  return bp_mixed_tiles(ctx, p, fbp_slice_shape(f, p, p.cachedSym, nView), ctx->scratch2.ptr, vc, nView, d_image,
+                        p.rotScale, true);
 }
 
 int ctsim_backprojector_mirror_members(const ctsim_backprojector* bp, const double* h_angles, int nView) {

@@ -400,4 +400,60 @@ MixedShape bp_default_shape(const BpPlan& p, int numCUs) {
   return m;
 }
 
+
+// By what was measured over sizes from 128 to 2048, the three geometries and
+// both interpolations (whole slices, FFT filter):
+//   rotated copies (the pipelined rotational kernel): 8 lanes along y, 2 rows
+//     per lane (1 up to 128^2); against the mirror kernel 94 / 132 us
+//     (equilinear 512^2 linear), 142 / 187 (equiangular 512^2 cubic), 385 / 404
+//     (parallel 1024^2 cubic), 2250 / 2254 (parallel 2048^2 linear);
+//   mirror partners (the mirror kernel): 8 lanes, 4 rows from 640^2 with
+//     linear interpolation, else 2 (1 with 16 lanes up to 128^2); against the
+//     plain kernel at its default 83 / 127 (equiangular 401^2), 1167 / 1635
+//     (parallel 2048^2, 1441 views);
+//   neither (the plain kernel): 8 lanes, 4 rows (16 lanes, 1 row up to 192^2):
+//     17 / 41 (128^2), 31 / 35 (256^2), 109 / 134 (512^2), 403 / 555 (1024^2)
+//     against 16 lanes, 4 rows and one group below 256 views.
+// View groups: 8, one per XCD, or 16 where the tiles are few; at least 8 views
+// each (4 base views of the rotational kernel).
+MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView) {
+  const bool cubic = p.interp == INTERP_CUBIC;
+  const size_t npix = static_cast<size_t>(p.nx) * p.ny;
+  auto side = [](int n, int t) { return (n + t - 1) / t; };
+  auto shape = [&](int lanesY, int P, int sym, int chunk) {
+    MixedShape m;
+    m.lanesY = lanesY; m.P = P; m.sym = sym; m.chunk = chunk;
+    m.W = bp_window_bound(p, 256 / lanesY, lanesY * P);
+    return m;
+  };
+  // groups over nx x ny pixels and `views` views, 16 below `few` tiles
+  auto groups = [&](MixedShape& m, int nx, int ny, int views, int few, int least) {
+    const int tiles = side(nx, 256 / m.lanesY) * side(ny, m.lanesY * m.P);
+    m.split = tiles < few ? 16 : 8;
+    while (m.split > 1 && views / m.split < least) m.split /= 2;
+  };
+  const bool tiny = npix <= static_cast<size_t>(128) * 128;
+  if (sv.S > 0) {
+    MixedShape m = shape(8, tiny ? 1 : 2, 2, 2);
+    if (bp_sym_ok_for(p, m, sv)) {
+      groups(m, p.nx / 2, p.nx / 2, nView / sv.S, 64, 4);
+      return m;
+    }
+  }
+  if (sv.NM >= 2) {
+    const bool rows4 = !cubic && npix >= static_cast<size_t>(640) * 640;
+    MixedShape m = tiny ? shape(16, 1, 3, 8) : shape(8, rows4 ? 4 : 2, 3, 8);
+    if (bp_mirror_chunk(p, m, sv.NM, nView) > 0) {
+      groups(m, side(p.nx, 2), sv.NM == 4 ? side(p.ny, 2) : p.ny, nView, 512, 8);
+      return m;
+    }
+  }
+  MixedShape m = npix <= static_cast<size_t>(192) * 192 ? shape(16, 1, 0, 16) : shape(8, 4, 0, 16);
+  const size_t view = static_cast<size_t>(m.W > 0 ? m.W : p.nDet + 4) * (cubic ? 16 : 8);
+  while (m.chunk > 4 && m.chunk * view > static_cast<size_t>(36) * 1024) m.chunk /= 2;
+  if (m.chunk * view > static_cast<size_t>(62) * 1024) return p.mixed;  // long windows: the default's staging
+  groups(m, p.nx, p.ny, nView, 1024, 8);
+  return m;
+}
+
 }  // namespace ctsim

@@ -105,8 +105,8 @@ struct BpPlan {
   // xs (ys) symmetric about 0: the Y (X) mirror maps pixel centres onto
   // pixel centres.
   bool mirX = false, mirY = false;
-  MixedShape mixed;                 // current launch shape (tuned or default)
-  bool mixedTuned = false;
+  MixedShape mixed;                 // the launch shape tuned or given, else the default
+  bool mixedTuned = false;          // mixed was tuned or given (else bp_auto_shape decides)
   // Per-view constants of the last angle set, kept on the device so repeated
   // reconstructions with the same views upload nothing.
   mutable std::vector<double> cachedAngles;
@@ -127,6 +127,9 @@ MirrorViews bp_view_consts_f32(const BpPlan& p, const double* angles, int nView,
 int bp_window_bound(const BpPlan& p, int tileX, int tileY);
 SymViews bp_sym_views(const double* angles, int nView);
 MixedShape bp_default_shape(const BpPlan& p, int numCUs);
+// The mixed launch shape of a plan that was neither tuned nor given one, for
+// views of this symmetry.
+MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView);
 
 // Device side (backproject.hip).
 int bp_upload_tables(BpPlan& p);
@@ -142,6 +145,9 @@ int bp_mixed_coef(ctsim_ctx* ctx, const BpPlan& p, const float* d_filtered, int 
 // The same into a caller buffer of nView * nDet coefficient records.
 int bp_mixed_coef_into(ctsim_ctx* ctx, const BpPlan& p, const float* d_filtered, int nView,
                        void* d_coef);
+// The mixed launch shape for these views: the plan's own when it was tuned or
+// given, else bp_auto_shape's.
+MixedShape bp_mixed_shape(const BpPlan& p, const SymViews& sv, int nView);
 // views: the symmetry of these angles (NULL: the plan's cached one);
 // partial: view-group partial images, split * nx * ny floats (NULL: the
 // context's scratch).

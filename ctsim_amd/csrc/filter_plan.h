@@ -59,6 +59,24 @@ int filter_launch_coef(ctsim_ctx* ctx, FilterPlan& p, const float* d_in, int nVi
 // power-of-two transform of at most 4096 points and no pre-interpolation.
 bool filter_can_coef(const FilterPlan& p);
 
+struct BpPlan;
+struct MixedShape;
+struct SymViews;
+
+// Scratch of one mixed slice: view constants, interval coefficients, filtered
+// rows and split projection values (convolution filters), view-group partial
+// images.
+struct SliceScratch {
+  size_t vc = 0, coef = 0, rows = 0, work = 0, partial = 0;
+  size_t total() const { return vc + coef + rows + work + partial; }
+};
+SliceScratch fbp_slice_scratch(const FilterPlan& f, const BpPlan& p, const MixedShape& m, int nView);
+// The launch shape of one mixed slice (backproject.hip): bp_mixed_shape's, or
+// the default where only with that one the slice fits the static scratch, so
+// that both slice entry points run one shape and the static one takes every
+// slice that the default fits.
+MixedShape fbp_slice_shape(const FilterPlan& f, const BpPlan& p, const SymViews& sv, int nView);
+
 }  // namespace ctsim
 
 struct ctsim_procsignal {

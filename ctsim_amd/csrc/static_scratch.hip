@@ -15,10 +15,8 @@
 // the kernels store in full before the combine reads them).
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cstring>
 #include <mutex>
-#include <vector>
+#include <string>
 
 #include "bp_plan.h"
 #include "filter_plan.h"
@@ -36,8 +34,6 @@ std::mutex g_mutex;                   // guards g_scratchPtr and g_vcHost
 void* g_scratchPtr[kMaxDevices] = {};  // device address of `scratch` per device
 // Host staging of the per-view constants (fixed capacity; no allocation).
 ViewConstF32 g_vcHost[kStaticMaxViews];
-
-size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace
 
@@ -80,34 +76,11 @@ extern "C" int ctsim_fbp_slice_static(ctsim_ctx* ctx, ctsim_procsignal* ps,
     if (ctx->device >= 0 && ctx->device < kMaxDevices) base = g_scratchPtr[ctx->device];
   }
   if (!base) return fail(CTSIM_ERR_INVALID, "ctsim_fbp_slice_static: static scratch not set up");
-  // Layout: view constants | interval coefficients | filtered rows and
-  // split projection values (convolution filters) | view-group partial
-  // images.
-  const bool cubic = p.interp == INTERP_CUBIC;
-  const size_t elem = cubic ? sizeof(float4) : sizeof(float2);
-  const bool coefFilter = filter_can_coef(f);
-  const MixedShape& m = p.mixed;
-  const int split = std::max(1, std::min(m.split, nView));
-  const size_t npix = static_cast<size_t>(p.nx) * p.ny;
-  const size_t vcBytes = align256(sizeof(ViewConstF32) * nView);
-  const size_t coefBytes = align256(static_cast<size_t>(nView) * p.nDet * elem);
-  const size_t rowBytes = coefFilter ? 0 : align256(static_cast<size_t>(nView) * f.n * sizeof(float));
-  const size_t workBytes = coefFilter ? 0 : align256(filter_work_bytes(f, CTSIM_PREC_MIXED, nView));
-  const size_t partBytes = split > 1 ? align256(static_cast<size_t>(split) * npix * sizeof(float)) : 0;
-  const size_t need = vcBytes + coefBytes + rowBytes + workBytes + partBytes;
-  if (need > kStaticScratchBytes)
-    return fail(CTSIM_ERR_INVALID,
-                "ctsim_fbp_slice_static: this slice needs " + std::to_string(need >> 20) +
-                    " MiB of scratch; the static array holds " +
-                    std::to_string(kStaticScratchBytes >> 20) + " MiB");
-  unsigned char* b = static_cast<unsigned char*>(base);
-  ViewConstF32* d_vc = reinterpret_cast<ViewConstF32*>(b);
-  void* d_coef = b + vcBytes;
-  float* d_rows = reinterpret_cast<float*>(b + vcBytes + coefBytes);
-  void* d_work = workBytes ? b + vcBytes + coefBytes + rowBytes : nullptr;
-  float* d_part = partBytes ? reinterpret_cast<float*>(b + vcBytes + coefBytes + rowBytes + workBytes) : nullptr;
   CTSIM_CHECK(ctx->activate());
   SymViews sv;
+  MixedShape m;
+  SliceScratch use;
+  unsigned char* const b = static_cast<unsigned char*>(base);
   {
     // the copy from pageable memory has read g_vcHost when it returns
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -115,10 +88,23 @@ extern "C" int ctsim_fbp_slice_static(ctsim_ctx* ctx, ctsim_procsignal* ps,
     sv = bp_sym_views(h_angles, nView);
     sv.NM = mv.NM;
     sv.mapO = mv.mapO;
-    CTSIM_HIP(hipMemcpyAsync(d_vc, g_vcHost, sizeof(ViewConstF32) * nView, hipMemcpyHostToDevice,
-                             ctx->stream));
+    m = fbp_slice_shape(f, p, sv, nView);
+    use = fbp_slice_scratch(f, p, m, nView);
+    if (use.total() > kStaticScratchBytes)
+      return fail(CTSIM_ERR_INVALID,
+                  "ctsim_fbp_slice_static: this slice needs " + std::to_string(use.total() >> 20) +
+                      " MiB of scratch; the static array holds " +
+                      std::to_string(kStaticScratchBytes >> 20) + " MiB");
+    CTSIM_HIP(hipMemcpyAsync(b, g_vcHost, sizeof(ViewConstF32) * nView, hipMemcpyHostToDevice, ctx->stream));
   }
-  if (coefFilter) {
+  // Layout: view constants | interval coefficients | filtered rows and split
+  // projection values (convolution filters) | view-group partial images.
+  const ViewConstF32* d_vc = reinterpret_cast<const ViewConstF32*>(b);
+  void* d_coef = b + use.vc;
+  float* d_rows = reinterpret_cast<float*>(b + use.vc + use.coef);
+  void* d_work = use.work ? b + use.vc + use.coef + use.rows : nullptr;
+  float* d_part = use.partial ? reinterpret_cast<float*>(b + use.vc + use.coef + use.rows + use.work) : nullptr;
+  if (filter_can_coef(f)) {
     CTSIM_CHECK(filter_launch_coef(ctx, f, d_sino, nView, d_coef, p.interp, p.kind == KIND_IDIFF));
   } else {
     CTSIM_CHECK(filter_launch(ctx, f, CTSIM_PREC_MIXED, d_sino, nView, d_rows, f.n, d_work));
