@@ -149,13 +149,7 @@ extern "C" int ctsim_phantom_rasterize(ctsim_ctx* ctx, ctsim_phantom* phm, int n
   if (nx < 2 || ny < 2) return fail(CTSIM_ERR_INVALID, "ctsim_phantom_rasterize: image smaller than 2x2");
   CTSIM_CHECK(ctx->activate());
   PhantomPlan& p = phm->plan;
-  if (p.dirty || !p.d_elems.ptr) {
-    CTSIM_CHECK(p.d_elems.reserve((p.elems.empty() ? 1 : p.elems.size()) * sizeof(ElemGPU)));
-    if (!p.elems.empty())
-      CTSIM_HIP(hipMemcpy(p.d_elems.ptr, p.elems.data(), p.elems.size() * sizeof(ElemGPU),
-                          hipMemcpyHostToDevice));
-    p.dirty = false;
-  }
+  CTSIM_CHECK(phantom_upload(p));
   if (nsample < 1) nsample = 1;
   // phantom.cpp:474-500
   const double dx = p.xmax - p.xmin, dy = p.ymax - p.ymin;

@@ -7,13 +7,15 @@
 // visit the same elements in the same order, so element data is read with
 // wave-uniform loads.  The detector and source positions are repeated sums
 // along the detector array (scanner.cpp:490-532); a first pass with one lane
-// per view performs that walk so every lane starts from the reference's
+// per sum performs that walk so every lane starts from the reference's
 // values.
 //
-//   F64 path    the reference's clipping step order: bounding-box reject by
-//               Cohen-Sutherland on the polygon outline's box, map to the
-//               element frame, circle clip by translate / rotate (atan2, cos,
-//               sin) / clamp / rotate back, map back, length.
+//   F64 path    short closed forms with error bounds for ellipses and
+//               rectangles, stored where the bounds round to one float32; the
+//               rest in the reference's clipping step order: bounding-box
+//               reject by Cohen-Sutherland on the polygon outline's box, map
+//               to the element frame, circle clip by translate / rotate
+//               (atan2, cos, sin) / clamp / rotate back, map back, length.
 //   mixed path  the same box reject, then closed-form FP64 chords for
 //               ellipses (quadratic in the element frame) and rectangles
 //               (slab clip); triangles, segments and sectors keep the
@@ -21,6 +23,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
+#include <vector>
 
 #include "crmath.h"
 #include "scan_plan.h"
@@ -55,65 +59,71 @@ __device__ __forceinline__ ViewSetup view_setup(const ViewEnds& e, int nDet, uns
 
 struct WalkArgs {
   const ViewEnds* ends;
-  double4* walk;  // [nView][nDet]: xs, ys, xd (or the detector angle), yd
-  int* counter;   // the ray-sum kernel's work counter, zeroed here
+  double4* walk;  // [nView][walk_row]
+  int* counter;   // the ray-sum kernels' three counters, zeroed here
   int nView, nDet, geom;
   unsigned nSample;
   double angDetInc, angDetLen;
 };
 
+// A view's row of the walk: the four increments, then xs, ys, xd (or the
+// detector angle) and yd of every kWalkStep-th detector.  A reader takes the
+// last steps itself.
+constexpr int kWalkStep = 4;
+__host__ __device__ inline int walk_row(int nDet) { return 1 + (nDet + kWalkStep - 1) / kWalkStep; }
+
 // The detector walk of projectSingleView (scanner.cpp:449-531): per view
-// four chains of rounded sums (xs, ys, and xd, yd or the detector angle),
-// one lane per chain, 16 views per block.  Each run of 64 detectors is
-// gathered in LDS and stored as whole rows of the walk.
+// four chains of rounded sums (xs, ys, and xd, yd or the detector angle), one
+// lane per chain, 16 views per block.
+//
+// What bounds it: the latency of the chains, nDet adds one after the other.
+// The stores go straight to memory, and only every kWalkStep-th state is kept:
+// with all of them (47 MB at 1440 views of 1024 detectors), gathered in LDS and
+// stored as rows between two barriers, each of which waits for the row's
+// stores, the kernel took 48 us there, now 11.
 constexpr int kWalkViews = 16;
-constexpr int kWalkRow = 64 * 4 + 4;  // doubles per view in LDS (padded against bank conflicts)
 __global__ __launch_bounds__(64) void raysum_walk_kernel(WalkArgs a) {
-  __shared__ double tile[kWalkViews * kWalkRow];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.counter = 0;
-  const int lane = threadIdx.x, vl = lane >> 2, comp = lane & 3, v0 = blockIdx.x * kWalkViews;
-  const int v = v0 + vl;
+  if (blockIdx.x == 0 && threadIdx.x < 3) a.counter[threadIdx.x] = 0;
+  const int lane = threadIdx.x, comp = lane & 3, v = blockIdx.x * kWalkViews + (lane >> 2);
+  if (v >= a.nView) return;
+  const ViewEnds e = a.ends[v];
+  const ViewSetup s = view_setup(e, a.nDet, a.nSample, a.geom, a.angDetInc);
+  const bool equi = a.geom == GEOM_EQUIANGULAR;
   double x = 0.0, inc = 0.0;
-  if (v < a.nView) {
-    const ViewEnds e = a.ends[v];
-    const ViewSetup s = view_setup(e, a.nDet, a.nSample, a.geom, a.angDetInc);
-    const bool equi = a.geom == GEOM_EQUIANGULAR;
-    if (comp == 0) { x = e.xs1 + (s.sdx / 2); inc = s.sdx; }
-    else if (comp == 1) { x = e.ys1 + (s.sdy / 2); inc = s.sdy; }
-    else if (comp == 2) {
-      if (equi) { x = e.detAngle - (a.angDetLen / 2) + s.aSampInc / 2; inc = s.aInc; }
-      else { x = e.xd1 + s.ddx2 / 2; inc = s.ddx; }
-    } else if (!equi) {  // yd (the equiangular walk keeps 0 here)
-      x = e.yd1 + s.ddy2 / 2;
-      inc = s.ddy;
-    }
+  if (comp == 0) { x = e.xs1 + (s.sdx / 2); inc = s.sdx; }
+  else if (comp == 1) { x = e.ys1 + (s.sdy / 2); inc = s.sdy; }
+  else if (comp == 2) {
+    if (equi) { x = e.detAngle - (a.angDetLen / 2) + s.aSampInc / 2; inc = s.aInc; }
+    else { x = e.xd1 + s.ddx2 / 2; inc = s.ddx; }
+  } else if (!equi) {  // yd (the equiangular walk keeps 0 here)
+    x = e.yd1 + s.ddy2 / 2;
+    inc = s.ddy;
   }
-  double* mine = tile + vl * kWalkRow + comp;
-  for (int d0 = 0; d0 < a.nDet; d0 += 64) {
-    const int n = min(64, a.nDet - d0);
-    if (n == 64) {  // a whole run: unrolled, the stores off the chain of adds
+  const int n = walk_row(a.nDet);
+  double* out = reinterpret_cast<double*>(a.walk + static_cast<size_t>(v) * n) + comp;
+  *out = inc;
+#pragma unroll 8
+  for (int c = 1; c < n; c++) {
+    out[4 * c] = x;
 #pragma unroll
-      for (int j = 0; j < 64; j++) {
-        mine[4 * j] = x;
-        x += inc;
-      }
-    } else {
-      for (int j = 0; j < n; j++) {
-        mine[4 * j] = x;
-        x += inc;
-      }
-    }
-    __syncthreads();
-    // row tv's cells tj, 64 lanes a round (n == 64: one view row per round)
-    for (int t = lane; t < kWalkViews * n; t += 64) {
-      const int tv = n == 64 ? t >> 6 : t / n, tj = n == 64 ? t & 63 : t - tv * n;
-      if (v0 + tv < a.nView) {
-        const double* c = tile + tv * kWalkRow + 4 * tj;
-        a.walk[static_cast<size_t>(v0 + tv) * a.nDet + d0 + tj] = make_double4(c[0], c[1], c[2], c[3]);
-      }
-    }
-    __syncthreads();
+    for (int j = 0; j < kWalkStep; j++) x += inc;
   }
+}
+
+// Detector d's state of view v's walk.
+__device__ __forceinline__ double4 walk_at(const double4* walk, int nDet, int v, int d) {
+  const double4* row = walk + static_cast<size_t>(v) * walk_row(nDet);
+  const double4 inc = row[0];
+  double4 w = row[1 + d / kWalkStep];
+#pragma unroll
+  for (int j = 1; j < kWalkStep; j++)
+    if (d % kWalkStep >= j) {
+      w.x += inc.x;
+      w.y += inc.y;
+      w.z += inc.z;
+      w.w += inc.w;
+    }
+  return w;
 }
 
 // --------------------------------------------------- reference clipping
@@ -448,18 +458,25 @@ struct RaysumArgs {
   const double4* walk;
   const ElemGPU* __restrict__ elems;
   float* sino;
-  int* counter;  // items taken so far (zeroed by the walk kernel)
+  int* counter;  // items taken so far, items and rays deferred (zeroed by the walk kernel)
   int nView, nDet, nElem, geom, storageOffset;
   unsigned nSample;
   double angDetInc, centerDetLength;
   int unitPulse;
+  // the short chord (fast = 0: every ray by the reference's chain) and what it
+  // defers: items (view, first detector) and single rays (view, detector)
+  const FastElem* __restrict__ fastElems;
+  int2* items;
+  int2* rays;
+  int fast, deferItems;  // deferItems: raysum_f64_kernel follows, for waves the short chord does not suit
+  double fastX, fastY, fastR, fastMin, fastFar;
 };
 
 // Detector end (a) and source end (b) of sample i of detector d's ray, as
 // raysum_ray walks them (to rounding: the hull test below has a margin).
 __device__ __forceinline__ void ray_ends(const RaysumArgs& a, const ViewSetup& s, int v, int d, unsigned i,
                                          double& ax, double& ay, double& bx, double& by) {
-  const double4 w = a.walk[static_cast<size_t>(v) * a.nDet + d];
+  const double4 w = walk_at(a.walk, a.nDet, v, d);
   bx = w.x;
   by = w.y;
   if (a.geom == GEOM_EQUIANGULAR) {
@@ -555,7 +572,7 @@ __device__ __forceinline__ unsigned long long uniform_u64(unsigned long long x) 
 __device__ __forceinline__ void raysum_ray(const RaysumArgs& a, const ViewSetup& s, int v, int d, bool active,
                                            const unsigned long long* masks, int nChunks, WaveQueue* qp) {
   const int lane = threadIdx.x;
-  const double4 w = a.walk[static_cast<size_t>(v) * a.nDet + (active ? d : a.nDet - 1)];
+  const double4 w = walk_at(a.walk, a.nDet, v, active ? d : a.nDet - 1);
   const double xs = w.x, ys = w.y;
   double xd = w.z, yd = w.w, ang = w.z;
   double sum = 0.0;
@@ -639,12 +656,252 @@ __device__ __forceinline__ void raysum_ray(const RaysumArgs& a, const ViewSetup&
   }
 }
 
-// A persistent wave per block takes items (view, 64 detectors) from a
-// counter until none is left: the rays' work differs widely (a ray through
-// the phantom's middle meets many elements), and taking items as waves free
-// up keeps every CU busy to the end.
+// ----------------------------------------------------- the short ray sum
+//
+// Only float(sum / nSample) of a ray is kept, so its chords are needed exactly
+// only when the sum lies within its error of a float32 rounding boundary.
+// This kernel sums short closed forms with bounds on their distance from the
+// reference's chain and stores a ray whose two bounds round to one float32
+// number; the others are deferred to raysum_rays_kernel, which runs the chain.
+// The result is the reference's bit for bit either way.
+//
+// Ellipse: the chord is 2 sqrt(A - (det c)^2) / A per unit of attenuation, A =
+// |M d|^2 for the ray's unit direction d and the linear map M onto the unit
+// circle, c the signed distance of its centre from the ray: about 40
+// instructions where the reference's clip takes an arc tangent, a sine, a
+// cosine and four rotations.  With z = t^2 = 1 - (det c)^2 / A, t the half
+// chord in the unit frame, against the reference's chain:
+//   z < -1e-6: the line passes the ellipse by far more than any rounding; the
+//     chain clips to zero;
+//   z > edge: the line cuts the polygon that the bounding box is taken from,
+//     so the box clip keeps it, and both chords are within
+//     80 u (max / min semi-axis) (ray end + centre + semi-axis) (1 + 1 / t) of
+//     the exact one (u = 2^-53).  The chain: 17 u T across (T the ends' size in
+//     the unit frame, at most (ray end + centre) / min; the transform's own
+//     rounding, the arc tangent's, sine's and cosine's and the rotation), hence
+//     17 u T / t in the half chord, twice, 14 u T for rotating, moving and
+//     mapping both ends back, all times the larger semi-axis; here 8 u of the
+//     centre's distance and 6 u aspect in A, 34 u / t in all;
+//   between: the ray is deferred.
+// Rectangle: the line's parameters at the four sides, each off by a
+// coordinate's error (64 u of the ends' size in the unit frame, both
+// evaluations) over the direction's component, give an interval that holds
+// the chord however the corners are decided; 80 u as above for mapping back.
+// Both ends of the ray must lie outside the disc that holds these elements, on
+// either side of it (the clip then replaces both), and T below 1e6 keeps the shares above far inside
+// the margins on z and in the chain's own tolerances.  The sums add in the same
+// order; their roundings are bounded by u times the elements times the sum of
+// the sizes, twice.  A wave that meets another type of element is deferred to
+// raysum_f64_kernel.
+//
+// What bounds it: FP64 VALU issue, two thirds of its cycles.  1440 views of 1024
+// detectors over 12 ellipses: the chain for every ray took 452 us, this kernel
+// takes 93 and raysum_rays_kernel 14 for the few rays that are deferred (calling
+// the chain from this kernel instead: 388 us, for the registers and the lanes
+// that wait).
+__device__ __forceinline__ double rcp_f64(double x) {
+  const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+
+// Element k's record, the same for the whole wave, through scalar loads.
+__device__ __forceinline__ FastElem load_fast(const FastElem* table, int k) {
+  typedef const __attribute__((address_space(4))) FastElem* Ptr;
+  const Ptr p = (Ptr)(reinterpret_cast<unsigned long long>(table)) + __builtin_amdgcn_readfirstlane(k);
+  FastElem f;
+  f.m[0] = p->m[0]; f.m[1] = p->m[1]; f.m[2] = p->m[2]; f.m[3] = p->m[3];
+  f.cx = p->cx; f.cy = p->cy; f.det2 = p->det2; f.att = p->att;
+  f.kappa = p->kappa; f.edge = p->edge; f.kind = p->kind;
+  return f;
+}
+
+__device__ __forceinline__ bool raysum_short(const RaysumArgs& a, const ViewSetup& s, int v, int d,
+                                             const unsigned long long* masks, int nChunks, float* out) {
+  const double4 w = walk_at(a.walk, a.nDet, v, d);
+  const double xs = w.x, ys = w.y;
+  double xd = w.z, yd = w.w, ang = w.z;
+  double sum = 0.0, size = 0.0;
+  float bound = 0.f;
+  bool sure = true;
+  for (unsigned i = 0; i < a.nSample; i++) {
+    if (a.geom == GEOM_EQUIANGULAR) {
+      double sa, ca;
+      crm_sincos(ang, &sa, &ca);
+      xd = a.centerDetLength * ca;
+      yd = a.centerDetLength * sa;
+    }
+    const double ddx = xs - xd, ddy = ys - yd, L = sqrt(ddx * ddx + ddy * ddy);
+    const double dx = ddx / L, dy = ddy / L;
+    // the ends lie outside the disc, on either side of it
+    const double fx = a.fastX - xd, fy = a.fastY - yd, sx = xs - a.fastX, sy = ys - a.fastY, R2 = a.fastR * a.fastR;
+    const double foot = fx * dx + fy * dy;
+    const double far = fmax(fabs(xd) + fabs(yd), fabs(xs) + fabs(ys)) + a.fastFar;
+    sure = sure && foot > 0.0 && L > foot && fx * fx + fy * fy > R2 && sx * sx + sy * sy > R2 && far < 1e6 * a.fastMin;
+    const float farf = static_cast<float>(far);
+    const double k0 = xd * dy - yd * dx;
+    float e = 0.f;
+    double rsum = 0.0;
+    // candidates newest first, the next one's record read ahead
+    int c = nChunks;
+    unsigned long long m = 0;
+    auto next = [&]() -> int {
+      while (!m) {
+        if (c == 0) return -1;
+        m = uniform_u64(masks[--c]);
+      }
+      const int b = 63 - __builtin_clzll(m);
+      m &= ~(1ull << b);
+      return 64 * c + b;
+    };
+    int kn = __builtin_amdgcn_readfirstlane(next());
+    if (kn >= 0) {
+      FastElem fn = load_fast(a.fastElems, kn);
+      while (kn >= 0) {
+        const FastElem f = fn;
+        kn = __builtin_amdgcn_readfirstlane(next());
+        if (kn >= 0) fn = load_fast(a.fastElems, kn);
+        const double qx = fma(dx, f.m[0], dy * f.m[2]), qy = fma(dx, f.m[1], dy * f.m[3]);
+        double chord = 0.0;
+        if (f.kind == 1) {
+          const double A = fma(qx, qx, qy * qy);
+          const double cr = fma(f.cy, dx, fma(-f.cx, dy, k0));
+          const double num = fma(-f.det2 * cr, cr, A);
+          if (!__any(num > -1e-6 * A)) continue;  // no lane's line comes near
+          const double inv = rcp_f64(A);
+          const float z = static_cast<float>(num * inv);
+          if (z > f.edge) {
+            // sqrt(num) by the hardware's reciprocal root and two steps
+            const double y = __builtin_amdgcn_rsq(num);
+            double g = num * y, h = 0.5 * y;
+            const double r1 = fma(-g, h, 0.5);
+            g = fma(g, r1, g);
+            h = fma(h, r1, h);
+            g = fma(fma(-g, g, num), h, g);
+            chord = g * inv * f.att;
+            e = fmaf(f.kappa, __builtin_amdgcn_rsqf(z), e);
+          } else if (!(z < -1e-6f)) {
+            sure = false;
+          }
+        } else {
+          const double px = fma(xd, f.m[0], fma(yd, f.m[2], f.cx)), py = fma(xd, f.m[1], fma(yd, f.m[3], f.cy));
+          const double ix = rcp_f64(qx), iy = rcp_f64(qy);
+          const double cx = -px * ix, cy = -py * iy, hx = fabs(ix), hy = fabs(iy);  // middles and half lengths
+          const double err = static_cast<double>(f.edge * farf), gx = err * hx, gy = err * hy;
+          const double in = fmin(cx + hx - gx, cy + hy - gy) - fmax(cx - hx + gx, cy - hy + gy);
+          const double ou = fmin(cx + hx + gx, cy + hy + gy) - fmax(cx - hx - gx, cy - hy - gy);
+          // a line along a side (or no number) is left to the chain
+          sure = sure && ou < 1e300 && hx < 1e12 * hy && hy < 1e12 * hx;
+          const double lo = fmax(in, 0.0), hi = fmax(ou, 0.0);
+          chord = 0.5 * (lo + hi) * f.att;
+          if (hi > 0.0) e += f.kappa + static_cast<float>(0.51 * (hi - lo) * fabs(f.att)) * __builtin_amdgcn_rcpf(farf);
+        }
+        rsum += chord;
+        size += fabs(chord);
+      }
+    }
+    sum += rsum;
+    bound = fmaf(e, farf, bound);
+    if (a.geom == GEOM_EQUIANGULAR) ang += s.aSampInc;
+    else { xd += s.ddx2; yd += s.ddy2; }
+  }
+  const double E = 1.01 * static_cast<double>(bound) + 2.5 * 0x1p-53 * (a.nElem + 2.0 + a.nSample) * size;
+  const float f0 = static_cast<float>((sum - E) / a.nSample), f1 = static_cast<float>((sum + E) / a.nSample);
+  *out = f0;
+  return sure & (__float_as_uint(f0) == __float_as_uint(f1)) & (f0 == f0);
+}
+
+// More unsure rays of a wave than this are cheaper 64 at a time, their pairs of
+// ray and element packed (raysum_f64_kernel), than a wave each.
+constexpr int kDeferRays = 8;
+
+// One wave per block and item (a view, 64 detectors).  The middle of the
+// detector comes first, over all views, its ends, whose rays meet few
+// elements, last: the short items fill the end of the launch.
+__global__ __launch_bounds__(64) void raysum_short_kernel(RaysumArgs a) {
+  __shared__ unsigned long long masks[kCandChunks];
+  const int blocks = (a.nDet + 63) / 64, nChunks = (a.nElem + 63) / 64;
+  const int ring = blockIdx.x / a.nView, v = static_cast<int>(blockIdx.x) - ring * a.nView;
+  const int d0 = 64 * (blocks / 2 + ((ring & 1) ? -((ring + 1) / 2) : ring / 2));
+  const int d = d0 + static_cast<int>(threadIdx.x), d1 = min(d0 + 63, a.nDet - 1);
+  const ViewSetup s = view_setup(a.ends[v], a.nDet, a.nSample, a.geom, a.angDetInc);
+  wave_candidates(a, s, v, d0, d1, masks, nChunks);
+  __syncthreads();
+  // an element of another type among the candidates
+  bool other = false;
+  for (int c = 0; c < nChunks; c++) {
+    const int k = 64 * c + static_cast<int>(threadIdx.x);
+    other = other || (((uniform_u64(masks[c]) >> threadIdx.x) & 1) && a.fastElems[k].kind == 0);
+  }
+  if (__any(other)) {
+    if (threadIdx.x == 0) a.items[atomicAdd(a.counter + 1, 1)] = make_int2(v, d0);
+    return;
+  }
+  float f;
+  const bool sure = raysum_short(a, s, v, min(d, a.nDet - 1), masks, nChunks, &f);
+  if (sure && d < a.nDet) a.sino[static_cast<size_t>(v + a.storageOffset) * a.nDet + d] = f;
+  const unsigned long long rest = __ballot(!sure && d < a.nDet);
+  if (__popcll(rest) > kDeferRays && a.deferItems) {
+    if (threadIdx.x == 0) a.items[atomicAdd(a.counter + 1, 1)] = make_int2(v, d0);
+  } else if (rest) {
+    int at = 0;
+    if (threadIdx.x == 0) at = atomicAdd(a.counter + 2, __popcll(rest));
+    at = __builtin_amdgcn_readfirstlane(at) + lanes_below(rest);
+    if ((rest >> threadIdx.x) & 1) a.rays[at] = make_int2(v, d);
+  }
+}
+
+// The deferred rays by the reference's chain, a wave per ray: lane k clips
+// element 64 c + k, and the chords are added in the element order.  One chain's
+// latency bounds it: a lane per ray would take an element's chain after the
+// other.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void raysum_rays_kernel(RaysumArgs a) {
+  const int nRays = a.counter[2], nChunks = (a.nElem + 63) / 64, lane = threadIdx.x;
+  for (int r = blockIdx.x; r < nRays; r += gridDim.x) {
+    const int2 at = a.rays[r];
+    const int v = __builtin_amdgcn_readfirstlane(at.x), d = __builtin_amdgcn_readfirstlane(at.y);
+    const ViewSetup s = view_setup(a.ends[v], a.nDet, a.nSample, a.geom, a.angDetInc);
+    const double4 w = walk_at(a.walk, a.nDet, v, d);
+    double xd = w.z, yd = w.w, ang = w.z, sum = 0.0;
+    for (unsigned i = 0; i < a.nSample; i++) {
+      if (a.geom == GEOM_EQUIANGULAR) {
+        double sa, ca;
+        crm_sincos(ang, &sa, &ca);
+        xd = a.centerDetLength * ca;
+        yd = a.centerDetLength * sa;
+      }
+      double rsum = 0.0;
+      for (int c = nChunks - 1; c >= 0; c--) {
+        const int k = 64 * c + lane;
+        const bool may = k < a.nElem && (a.elems[k].type == PE_ELLIPSE
+                                             ? line_may_hit_unit_circle(a.elems[k].p2o, xd, yd, w.x, w.y)
+                                             : seg_may_hit_box(xd, yd, w.x, w.y, a.elems[k].lim));
+        double chord = 0.0;
+        if (may) chord = chord_ref(a.elems[k], xd, yd, w.x, w.y);
+        unsigned long long m = __ballot(may);
+        const unsigned long long bits = __builtin_bit_cast(unsigned long long, chord);
+        while (m) {  // newest first
+          const int b = 63 - __builtin_clzll(m);
+          m &= ~(1ull << b);
+          const unsigned hi = __builtin_amdgcn_readlane(static_cast<int>(bits >> 32), b);
+          const unsigned lo = __builtin_amdgcn_readlane(static_cast<int>(bits), b);
+          rsum += __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
+        }
+      }
+      sum += rsum;
+      if (a.geom == GEOM_EQUIANGULAR) ang += s.aSampInc;
+      else { xd += s.ddx2; yd += s.ddy2; }
+    }
+    if (lane == 0) a.sino[static_cast<size_t>(v + a.storageOffset) * a.nDet + d] = static_cast<float>(sum / a.nSample);
+  }
+}
+
+// A persistent wave per block takes items (view, 64 detectors; of those that
+// raysum_short_kernel deferred, where it ran) from a counter until none is
+// left: the rays' work differs widely (a ray through the phantom's middle meets
+// many elements), and taking items as waves free up keeps every CU busy to the
+// end.
 __device__ __forceinline__ void raysum_items(const RaysumArgs& a, WaveQueue* q) {
-  const int blocks = (a.nDet + 63) / 64, nItems = blocks * a.nView;
+  const int blocks = (a.nDet + 63) / 64, nItems = a.fast ? a.counter[1] : blocks * a.nView;
   const int nChunks = (a.nElem + 63) / 64;
   const bool cull = nChunks <= kCandChunks;
   __shared__ unsigned long long masks[kCandChunks];  // the wave's candidate masks
@@ -653,7 +910,12 @@ __device__ __forceinline__ void raysum_items(const RaysumArgs& a, WaveQueue* q) 
     if (threadIdx.x == 0) item = atomicAdd(a.counter, 1);
     item = __builtin_amdgcn_readfirstlane(item);
     if (item >= nItems) break;
-    const int v = item / blocks, d0 = (item - v * blocks) * 64;
+    int v = item / blocks, d0 = (item - v * blocks) * 64;
+    if (a.fast) {
+      const int2 r = a.items[item];
+      v = __builtin_amdgcn_readfirstlane(r.x);
+      d0 = __builtin_amdgcn_readfirstlane(r.y);
+    }
     const int d = d0 + static_cast<int>(threadIdx.x), d1 = min(d0 + 63, a.nDet - 1);
     if (a.unitPulse) {  // scanner.cpp:475-478
       if (d < a.nDet) a.sino[static_cast<size_t>(v + a.storageOffset) * a.nDet + d] = d == a.nDet / 2 ? 1.f : 0.f;
@@ -686,7 +948,7 @@ __global__ __launch_bounds__(256) void raysum_closed_kernel(RaysumArgs a) {
     return;
   }
   const ViewSetup s = view_setup(a.ends[v], a.nDet, a.nSample, a.geom, a.angDetInc);
-  const double4 w = a.walk[static_cast<size_t>(v) * a.nDet + d];
+  const double4 w = walk_at(a.walk, a.nDet, v, d);
   const double xs = w.x, ys = w.y;
   double xd = w.z, yd = w.w, ang = w.z;
   double sum = 0.0;
@@ -709,17 +971,27 @@ __global__ __launch_bounds__(256) void raysum_closed_kernel(RaysumArgs a) {
 
 }  // namespace
 
+int phantom_upload(PhantomPlan& p) {
+  if (!p.dirty && p.d_elems.ptr) return CTSIM_OK;
+  const size_t n = p.elems.size();
+  CTSIM_CHECK(p.d_elems.reserve((n ? n : 1) * (sizeof(ElemGPU) + sizeof(FastElem))));
+  if (n) {
+    std::vector<unsigned char> all(n * (sizeof(ElemGPU) + sizeof(FastElem)));
+    const std::vector<FastElem> fast = phantom_fast_elems(p);
+    memcpy(all.data(), p.elems.data(), n * sizeof(ElemGPU));
+    memcpy(all.data() + n * sizeof(ElemGPU), fast.data(), n * sizeof(FastElem));
+    CTSIM_HIP(hipMemcpy(p.d_elems.ptr, all.data(), all.size(), hipMemcpyHostToDevice));
+  }
+  p.dirty = false;
+  return CTSIM_OK;
+}
+
 int raysum_launch(ctsim_ctx* ctx, const ScannerPlan& s, PhantomPlan& p, int precision,
                   int iStartView, int iNumViews, int iOffsetView, int iStorageOffset,
                   float* d_sino, double* h_angles) {
   if (iNumViews <= 0) return CTSIM_OK;
   const hipStream_t st = ctx->stream;
-  if (p.dirty || !p.d_elems.ptr) {
-    CTSIM_CHECK(p.d_elems.reserve(p.elems.size() * sizeof(ElemGPU)));
-    CTSIM_HIP(hipMemcpy(p.d_elems.ptr, p.elems.data(), p.elems.size() * sizeof(ElemGPU),
-                        hipMemcpyHostToDevice));
-    p.dirty = false;
-  }
+  CTSIM_CHECK(phantom_upload(p));
   const size_t eb = static_cast<size_t>(iNumViews) * sizeof(ViewEnds);
   CTSIM_CHECK(ctx->stage.reserve(eb, st));
   ViewEnds* ends = static_cast<ViewEnds*>(ctx->stage.ptr);
@@ -727,27 +999,50 @@ int raysum_launch(ctsim_ctx* ctx, const ScannerPlan& s, PhantomPlan& p, int prec
   if (h_angles)
     for (int v = 0; v < iNumViews; v++) h_angles[v + iStorageOffset] = ends[v].viewAngle;
   CTSIM_CHECK(ctx->stage.upload(ctx->viewConsts, eb, st));
-  // the walk, then the ray-sum kernel's work counter
-  const size_t walkBytes = static_cast<size_t>(iNumViews) * s.nDet * sizeof(double4);
-  CTSIM_CHECK(ctx->scratch.reserve(walkBytes + 256));
+  // the walk, the ray-sum kernels' counters, what the short chord defers
+  const size_t walkBytes = static_cast<size_t>(iNumViews) * walk_row(s.nDet) * sizeof(double4);
+  const int items = ((s.nDet + 63) / 64) * iNumViews;
+  const size_t rays = static_cast<size_t>(iNumViews) * s.nDet;
+  // The short chord is for phantoms with an element that it knows and whose
+  // size against the scan leaves its bound room (else every ray is deferred).
+  const double rim = std::max({hypot(s.xs1, s.ys1), hypot(s.xs2, s.ys2), hypot(s.xd1, s.yd1), hypot(s.xd2, s.yd2),
+                               s.centerDetLength});
+  const bool fast = precision == CTSIM_PREC_F64 && !p.unitPulse && p.elems.size() <= 64 * kCandChunks &&
+                    p.fastR > 0 && 1.5 * rim + p.fastFar < 1e6 * p.fastMin;
+  // Whole items are deferred where other types are met or a ray may end in the
+  // elements' disc.
+  const bool deferItems = p.fastOthers || !(std::min(s.focalLength, s.centerDetLength) >
+                                            1.001 * (hypot(p.fastX - s.xc, p.fastY - s.yc) + p.fastR));
+  CTSIM_CHECK(ctx->scratch.reserve(walkBytes + 256 + (fast ? (items + rays) * sizeof(int2) : 0)));
   int* counter = reinterpret_cast<int*>(static_cast<unsigned char*>(ctx->scratch.ptr) + walkBytes);
   WalkArgs wa{ctx->viewConsts.as<ViewEnds>(), ctx->scratch.as<double4>(), counter, iNumViews, s.nDet,
               s.geom, s.nSample, s.angDetInc, s.angDetLen};
   hipLaunchKernelGGL(raysum_walk_kernel, dim3((iNumViews + kWalkViews - 1) / kWalkViews), dim3(64), 0, st, wa);
   CTSIM_HIP(hipGetLastError());
+  int2* deferred = reinterpret_cast<int2*>(reinterpret_cast<unsigned char*>(counter) + 256);
   RaysumArgs ra{ctx->viewConsts.as<ViewEnds>(), ctx->scratch.as<double4>(), p.d_elems.as<ElemGPU>(),
                 d_sino, counter, iNumViews, s.nDet, static_cast<int>(p.elems.size()), s.geom, iStorageOffset,
-                s.nSample, s.angDetInc, s.centerDetLength, p.unitPulse ? 1 : 0};
+                s.nSample, s.angDetInc, s.centerDetLength, p.unitPulse ? 1 : 0,
+                reinterpret_cast<const FastElem*>(p.d_elems.as<ElemGPU>() + p.elems.size()), deferred, deferred + items,
+                fast ? 1 : 0, deferItems ? 1 : 0, p.fastX, p.fastY, p.fastR, p.fastMin, p.fastFar};
   if (precision == CTSIM_PREC_F64) {
     // persistent single-wave blocks, as many as are resident at once, no
     // more than the items
-    const int items = ((s.nDet + 63) / 64) * iNumViews;
-    int perCU = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, reinterpret_cast<const void*>(raysum_f64_kernel), 64,
-                                                     0) != hipSuccess ||
-        perCU < 1)
-      perCU = 8;
-    hipLaunchKernelGGL(raysum_f64_kernel, dim3(std::min(items, ctx->numCUs * perCU)), dim3(64), 0, st, ra);
+    auto resident = [&](auto kern, int n) {
+      int perCU = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, reinterpret_cast<const void*>(kern), 64, 0) != hipSuccess ||
+          perCU < 1)
+        perCU = 8;
+      return dim3(static_cast<unsigned>(std::min(n, ctx->numCUs * perCU)));
+    };
+    if (fast) {
+      hipLaunchKernelGGL(raysum_short_kernel, dim3(items), dim3(64), 0, st, ra);
+      CTSIM_HIP(hipGetLastError());
+      hipLaunchKernelGGL(raysum_rays_kernel, resident(raysum_rays_kernel, items), dim3(64), 0, st, ra);
+      CTSIM_HIP(hipGetLastError());
+    }
+    if (!fast || deferItems)
+      hipLaunchKernelGGL(raysum_f64_kernel, resident(raysum_f64_kernel, items), dim3(64), 0, st, ra);
   } else {
     hipLaunchKernelGGL(raysum_closed_kernel, dim3((s.nDet + 255) / 256, iNumViews), dim3(256), 0, st, ra);
   }

@@ -176,6 +176,58 @@ int phantom_add(PhantomPlan& p, const char* typeName, double cx, double cy, doub
   return CTSIM_OK;
 }
 
+// The bounds' constants: 80 roundings (u = 2^-53) of the element's aspect
+// times the scan's size in a chord (an ellipse's over its half chord, doubled
+// for 1 + 1 / t <= 2 / t), 64 of a coordinate in the unit frame; raysum.hip
+// counts them.
+std::vector<FastElem> phantom_fast_elems(PhantomPlan& p) {
+  std::vector<FastElem> out(p.elems.size());
+  p.fastX = 0.5 * (p.xmin + p.xmax);
+  p.fastY = 0.5 * (p.ymin + p.ymax);
+  p.fastR = 0;
+  p.fastMin = 1e300;
+  p.fastFar = 0;
+  p.fastOthers = false;
+  for (size_t k = 0; k < p.elems.size(); k++) {
+    const ElemGPU& e = p.elems[k];
+    const ElemInfo& in = p.infos[k];
+    FastElem& f = out[k];
+    f = FastElem{};
+    const bool ellipse = e.type == PE_ELLIPSE;
+    const double lo = fmin(in.u, in.v), hi = fmax(in.u, in.v);
+    const double reach = ellipse ? hi : sqrt(in.u * in.u + in.v * in.v);
+    if (!(ellipse || e.type == PE_RECT) || !(lo > 0) || !(hi / lo < 1e4) || !(fabs(in.atten) < 1e30) ||
+        (ellipse && in.nOutline < 32) || !(fabs(in.cx) + fabs(in.cy) + reach < 1e30)) {
+      p.fastOthers = true;
+      continue;
+    }
+    for (int q = 0; q < 4; q++) f.m[q] = e.p2o[q];
+    const double u = 0x1p-53 * 1.0001;
+    f.kappa = static_cast<float>((ellipse ? 2 : 1) * 80 * u * fabs(in.atten) * hi / lo);
+    if (ellipse) {
+      const double det = e.p2o[0] * e.p2o[3] - e.p2o[1] * e.p2o[2], c = cos(kPi / (in.nOutline - 1));
+      f.det2 = det * det;
+      f.cx = in.cx;
+      f.cy = in.cy;
+      f.att = 2 * in.atten;
+      f.edge = static_cast<float>(1 - c * c + 2e-6);
+      f.kind = 1;
+    } else {
+      f.cx = e.p2o[4];
+      f.cy = e.p2o[5];
+      f.att = in.atten;
+      f.edge = static_cast<float>(64 * u / lo);
+      f.kind = 2;
+    }
+    const double dx = in.cx - p.fastX, dy = in.cy - p.fastY;
+    p.fastR = fmax(p.fastR, sqrt(dx * dx + dy * dy) + reach);
+    p.fastMin = fmin(p.fastMin, lo);
+    p.fastFar = fmax(p.fastFar, sqrt(in.cx * in.cx + in.cy * in.cy) + reach);
+  }
+  p.fastR *= 1 + 1e-6;
+  return out;
+}
+
 // Phantom::createFromPhantom, addStdHerman, addStdSheppLogan,
 // phantom.cpp:128-170, 390-433
 int phantom_builtin(PhantomPlan& p, const char* name) {

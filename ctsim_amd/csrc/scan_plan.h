@@ -30,13 +30,32 @@ struct ElemInfo {
   double rotDeg;  // the rotation as defined
 };
 
+// What the FP64 ray sums' short chord needs of an ellipse or a rectangle
+// (raysum.hip); kind is 0 for the other types and for elements outside its
+// error bound's range.
+struct FastElem {
+  double m[4];    // phantom -> unit frame, linear part (p2o[0..3])
+  double cx, cy;  // ellipse: centre; rectangle: p2o[4], p2o[5]
+  double det2;    // ellipse: determinant of the linear part, squared
+  double att;     // attenuation (ellipse: twice)
+  float kappa;    // error bound of a chord, per unit of scan size
+  float edge;     // ellipse: half chords squared below this may miss the outline polygon's box
+                  // rectangle: error of a coordinate in the unit frame, per unit of scan size
+  int kind;       // 1 ellipse, 2 rectangle
+  int pad;
+};
+
 struct PhantomPlan {
   std::vector<ElemGPU> elems;  // definition order (the reference's list is newest-first)
   std::vector<ElemInfo> infos; // same order as elems
   double xmin = 1E30, xmax = -1E30, ymin = 1E30, ymax = -1E30;
   bool unitPulse = false;
-  DevBuf d_elems;
+  DevBuf d_elems;              // ElemGPU per element, then FastElem per element
   bool dirty = true;
+  // Of the elements with a short chord: a disc about the extent's centre that
+  // holds them, the smallest semi-axis, the largest |centre| + semi-axis
+  double fastX = 0, fastY = 0, fastR = 0, fastMin = 1e300, fastFar = 0;
+  bool fastOthers = false;  // there are elements without one
 };
 
 struct ScannerPlan {
@@ -64,6 +83,10 @@ int scanner_init(ScannerPlan& s, const PhantomPlan& p, const char* geometry, int
 void scanner_view_ends(const ScannerPlan& s, int iStartView, int iNumViews, int iOffsetView,
                        ViewEnds* out);
 
+// FastElem of every element, and the plan's summary of them.
+std::vector<FastElem> phantom_fast_elems(PhantomPlan& p);
+// Uploads the elements if they changed.
+int phantom_upload(PhantomPlan& p);
 int raysum_launch(ctsim_ctx* ctx, const ScannerPlan& s, PhantomPlan& p, int precision,
                   int iStartView, int iNumViews, int iOffsetView, int iStorageOffset,
                   float* d_sino, double* h_angles);
