@@ -17,14 +17,15 @@
 // Slices are dealt to the 8 XCDs by longest-processing-time first, so a
 // slice's coefficients are produced and consumed under one L2; a slice that
 // costs more than 1/32 of the batch is dealt item by item over all eight.
-// Each XCD has its own queue (its filter items, then its BP items, largest
-// slices first); workgroups pull items from their XCD's queue with an
-// atomic counter.  A BP item waits (bounded spin, error flag on expiry)
-// until its slice's filter items are done.  Filter items never wait, and in
-// every queue they precede all BP items, so by the time a workgroup takes a
-// BP item every filter item of its queue has been taken by a running
-// workgroup; each filter item a BP item can wait on (in any queue) is
-// therefore finished or held by a running workgroup, and the wait ends.
+// Each XCD has its own queue (its filter items, then its BP items, longest
+// first); workgroups pull items from their XCD's queue with an atomic counter,
+// and from the others' once it is drained.  A BP item waits (bounded spin,
+// error flag on expiry) until its slice's filter items are done.  Filter items
+// never wait, and in every queue they precede all BP items, so by the time a
+// workgroup takes a BP item every filter item of that queue has been taken by a
+// running workgroup; another queue's filter items are taken at the latest by
+// that queue's own workgroups, which wait on nothing before them, and so the
+// wait ends.
 // Fused mode runs both item kinds in one launch; two-phase mode launches
 // the filter items and then the BP items (no waiting, smaller LDS for the
 // BP launch).  The autotuner picks the mode, the tile shape, the views per
@@ -213,7 +214,71 @@ __device__ __forceinline__ void filter_item(const SliceDev& s, int pair, Cplx<fl
   }
 }
 
-// counters: [0, 8) queue heads, [8, 8 + nSlices) filter items done per slice.
+// Queue heads lie this many counters apart: workgroups of all XCDs update
+// them, and heads on one cache line wait for each other (1850 filter items of
+// 1024 points: 82 us with the heads side by side and every item from one, 45).
+constexpr int kHead = 32;
+
+// The next item for a workgroup, or -1 when all eight queues are drained;
+// called by the whole workgroup, between barriers that protect s_item.  RANKED:
+// its first item is its rank in its own queue, the others come from the head,
+// which counts on from the ranks (not for items that others wait for: a
+// workgroup may start late).  Once its own queue is drained it takes from the
+// others that still hold items, starting at another one per workgroup, so that
+// no XCD idles while another has work (16 slices of three geometries, the
+// queues in order of slice cost: a quarter of the CU cycles idle in 1640 us of
+// backprojection; taking from others, longest items first, 1500 us).  The heads
+// only grow, so every workgroup ends.
+template <bool RANKED>
+struct ItemQueue {
+  const int* start;  // of the eight queues and the end
+  int* heads;
+  int own, rank;  // own queue (-1: drained), workgroup of it
+  bool first = RANKED;
+  __device__ __forceinline__ ItemQueue(const int* queueStart, int* h)
+      : start(queueStart), heads(h), own(blockIdx.x & 7), rank(blockIdx.x >> 3) {}
+  __device__ __forceinline__ int taken(int t) const { return start[t] + (RANKED ? gridDim.x >> 3 : 0); }
+  __device__ __forceinline__ int next(int* s_item) {
+    if (threadIdx.x < 64) {
+      int item = -1;
+      if (own >= 0) {
+        if (first) item = start[own] + rank;
+        else if (threadIdx.x == 0) item = taken(own) + atomicAdd(&heads[kHead * own], 1);
+        first = false;
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item >= start[own + 1]) {
+          own = -1;
+          item = -1;
+        }
+      }
+      if (item < 0) {
+        const int r = (rank + static_cast<int>(threadIdx.x & 7)) & 7;
+        const int left = start[r + 1] - taken(r) -
+                         __hip_atomic_load(&heads[kHead * r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned rest = static_cast<unsigned>(__ballot(left > 0)) & 0xffu;
+        while (rest && item < 0) {
+          const int t = (rank + __builtin_ctz(rest)) & 7;
+          rest &= rest - 1;
+          if (threadIdx.x == 0) item = taken(t) + atomicAdd(&heads[kHead * t], 1);
+          item = __builtin_amdgcn_readfirstlane(item);
+          if (item >= start[t + 1]) item = -1;
+        }
+      }
+      if (threadIdx.x == 0) *s_item = item;
+    }
+    return broadcast(s_item);
+  }
+  __device__ __forceinline__ int broadcast(const int* s_item) {
+    __syncthreads();
+    // wave-uniform, so the item and its slice descriptor load into scalar
+    // registers instead of occupying vector registers in every lane
+    const int i = __builtin_amdgcn_readfirstlane(*s_item);
+    __syncthreads();
+    return i;
+  }
+};
+
+// counters: the eight queue heads, then the filter items done per slice.
 // SYM instantiates the symmetric body (P <= 2); the plain kernel leaves it
 // out and keeps its own register budget.  DO_F / DO_B instantiate the filter
 // and the backprojection items: the fused launch takes both, the two-phase
@@ -235,17 +300,11 @@ __device__ __forceinline__ void fbp_batch_body(const SliceDev* __restrict__ slic
   float4* s_v = s_meta;
   dev::SymWin* s_win = reinterpret_cast<dev::SymWin*>(s_meta);
   float2* s_ab = reinterpret_cast<float2*>(s_meta + 256);
-  const int q = blockIdx.x & 7;
-  const int qBegin = queueStart[q], qEnd = queueStart[q + 1];
-  int* done = counters + 8;
+  ItemQueue<!(DO_F && DO_B)> queue(queueStart, counters);
+  int* done = counters + 8 * kHead;
   while (true) {
-    if (threadIdx.x == 0) s_item = qBegin + atomicAdd(&counters[q], 1);
-    __syncthreads();
-    // wave-uniform, so the item and its slice descriptor load into scalar
-    // registers instead of occupying vector registers in every lane
-    const int i = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();
-    if (i >= qEnd) break;  // every workgroup ends when its queue is drained
+    const int i = queue.next(&s_item);
+    if (i < 0) break;
     const Item it = items[i];
     const SliceDev& s = slices[it.slice];
     if (it.kind == kFilterItem) {
@@ -368,14 +427,10 @@ __global__ __launch_bounds__(256) void fbp_batch_sym_class_kernel(const SliceDev
   __shared__ dev::SymWin s_win[256];
   __shared__ float2 s_ab[64];
   __shared__ int s_item;
-  const int q = blockIdx.x & 7;
-  const int qBegin = queueStart[q], qEnd = queueStart[q + 1];
+  ItemQueue<true> queue(queueStart, counters);
   while (true) {
-    if (threadIdx.x == 0) s_item = qBegin + atomicAdd(&counters[q], 1);
-    __syncthreads();
-    const int i = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();
-    if (i >= qEnd) break;  // every workgroup ends when its queue is drained
+    const int i = queue.next(&s_item);
+    if (i < 0) break;
     const Item it = items[i];
     const SliceDev& s = slices[it.slice];
     dev::bp_sym_tile_pipe<GK, INTERP, P, DEG, S, K>(s.bp, it.a, it.pad,
@@ -415,14 +470,10 @@ __global__ __launch_bounds__(256) void fbp_batch_plain_class_kernel(const SliceD
   __shared__ float4 s_v[dev::kMaxChunk + 2];
   __shared__ int s_lo[dev::kMaxChunk];
   __shared__ int s_item;
-  const int q = blockIdx.x & 7;
-  const int qBegin = queueStart[q], qEnd = queueStart[q + 1];
+  ItemQueue<true> queue(queueStart, counters);
   while (true) {
-    if (threadIdx.x == 0) s_item = qBegin + atomicAdd(&counters[q], 1);
-    __syncthreads();
-    const int i = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();
-    if (i >= qEnd) break;  // every workgroup ends when its queue is drained
+    const int i = queue.next(&s_item);
+    if (i < 0) break;
     const Item it = items[i];
     const SliceDev& s = slices[it.slice];
     if constexpr (NM > 1)
@@ -598,11 +649,13 @@ void launch_filter_class(const ctsim_batch& b, const ctsim_batch::FilterClass& f
   }
 }
 
-// counters: [0, 8) the fused launch's queue heads, [8, 8 + nSlices) its filter
-// items done per slice, then 8 queue heads for each two-phase launch (filter
-// classes, then backprojection classes), all zeroed by one reset kernel.
+// counters: the fused launch's 8 queue heads, its filter items done per slice,
+// then (from the next multiple of kHead) 8 queue heads for each two-phase
+// launch (filter classes, then backprojection classes), all zeroed by one reset
+// kernel.
+size_t batch_heads(const ctsim_batch& b) { return 8 * kHead + (b.s.size() + kHead - 1) / kHead * kHead; }
 size_t batch_counters(const ctsim_batch& b) {
-  return 8 + b.s.size() + 8 * (b.fclass.size() + b.bclass.size());
+  return batch_heads(b) + 8 * kHead * (b.fclass.size() + b.bclass.size());
 }
 
 // The symmetric instantiation runs when some slice takes the symmetric body.
@@ -719,12 +772,12 @@ int batch_layout(ctsim_ctx* ctx, ctsim_batch& b) {
     a.split = 1;
     a.viewsPerGroup = p.nView;
     a.center = static_cast<float>(p.iDetCenter);
-    a.F = static_cast<float>(p.F);
-    a.twoF = static_cast<float>(2 * p.F);
     a.endScale = static_cast<float>(p.rotScale);
-    a.posScale = d.gk == 2 ? static_cast<float>(p.sdl / p.detInc) : static_cast<float>(1.0 / p.detInc);
     if (d.deg > 0) for (int j = 0; j <= d.deg; j++) a.atan[j] = p.atanCoef[j];
     else a.atan[0] = static_cast<float>(1.0 / p.detInc);
+    a.F = static_cast<float>(p.F);
+    a.twoF = static_cast<float>(2 * p.F);
+    a.posScale = d.gk == 2 ? static_cast<float>(p.sdl / p.detInc) : static_cast<float>(1.0 / p.detInc);
     a.xs = p.d_xy.as<float>();
     a.ys = p.d_xy.as<float>() + p.xs.size();
     a.vc = sl.vc.as<ViewConstF32>();
@@ -802,6 +855,14 @@ int batch_layout(ctsim_ctx* ctx, ctsim_batch& b) {
       load[x] += b.s[k].cost;
     }
   }
+  // in each queue the items that take longest first (a long one taken last
+  // keeps one workgroup busy while the others have none left)
+  auto itemCost = [&](const Item& it) {
+    const SliceDev& d = b.host[it.slice];
+    return b.s[it.slice].cost / (static_cast<double>(d.bp.tilesX) * d.bp.tilesY * (d.sym ? d.bp.split : 1));
+  };
+  for (auto& q : bpq)
+    std::stable_sort(q.begin(), q.end(), [&](const Item& x, const Item& y) { return itemCost(x) > itemCost(y); });
   // the two-phase filter launches by transform length class
   std::vector<Item> itemsFc;
   std::vector<int> qFc;
@@ -956,8 +1017,8 @@ void launch_batch(ctsim_batch& b, hipStream_t st) {
   } else {
     // one filter launch per transform length class, then one backprojection
     // launch per class, each with queue heads of its own
-    int* heads = b.d_counters.as<int>() + 8 + S;
-    for (size_t c = 0; c < b.fclass.size(); c++, heads += 8) launch_filter_class(b, b.fclass[c], heads, st);
+    int* heads = b.d_counters.as<int>() + batch_heads(b);
+    for (size_t c = 0; c < b.fclass.size(); c++, heads += 8 * kHead) launch_filter_class(b, b.fclass[c], heads, st);
     for (const auto& bc : b.bclass) {
       const SliceDev* sl = b.d_slices.as<SliceDev>();
       const Item* it = b.d_itemsBc.as<Item>();
@@ -966,7 +1027,7 @@ void launch_batch(ctsim_batch& b, hipStream_t st) {
       int* e = b.d_error.as<int>();
       void* args[] = {&sl, &it, &q, &c, &e};
       (void)hipLaunchKernel(bc.kernel, dim3(bc.grid), dim3(256), args, bc.lds, st);
-      heads += 8;
+      heads += 8 * kHead;
     }
   }
   if (b.nCombine > 0)

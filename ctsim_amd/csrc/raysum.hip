@@ -695,10 +695,10 @@ __device__ __forceinline__ void raysum_ray(const RaysumArgs& a, const ViewSetup&
 // raysum_f64_kernel.
 //
 // What bounds it: FP64 VALU issue, two thirds of its cycles.  1440 views of 1024
-// detectors over 12 ellipses: the chain for every ray took 452 us, this kernel
-// takes 93 and raysum_rays_kernel 14 for the few rays that are deferred (calling
-// the chain from this kernel instead: 388 us, for the registers and the lanes
-// that wait).
+// detectors over 64 ellipses and 4 rectangles: the chain for every ray took
+// 452 us, this kernel takes 93 and raysum_rays_kernel 14 for the few rays that
+// are deferred (calling the chain from this kernel instead: 388 us, for the
+// registers and the lanes that wait).
 __device__ __forceinline__ double rcp_f64(double x) {
   const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
   return fma(r, fma(e, e, e), r);
