@@ -637,10 +637,15 @@ int bp_upload_tables(BpPlan& p) {
     CTSIM_HIP(hipMemcpy(p.d_rphi.as<double>() + 2 * n, xy.data(), xy.size() * sizeof(double),
                         hipMemcpyHostToDevice));
   }
-  CTSIM_CHECK(p.d_xy.reserve((p.xs.size() + p.ys.size()) * sizeof(float)));
-  CTSIM_HIP(hipMemcpy(p.d_xy.ptr, p.xs.data(), p.xs.size() * sizeof(float), hipMemcpyHostToDevice));
-  CTSIM_HIP(hipMemcpy(p.d_xy.as<float>() + p.xs.size(), p.ys.data(), p.ys.size() * sizeof(float),
-                      hipMemcpyHostToDevice));
+  std::vector<float> xyf(p.xs);
+  xyf.insert(xyf.end(), p.ys.begin(), p.ys.end());
+  if (p.geom == GEOM_EQUILINEAR)  // and in units of the focal length, in detector cells at the centre
+    for (double scale : {1.0, p.sdl / p.detInc}) {
+      for (double x : p.xd) xyf.push_back(static_cast<float>(x / p.F * scale));
+      for (double y : p.yd) xyf.push_back(static_cast<float>(y / p.F * scale));
+    }
+  CTSIM_CHECK(p.d_xy.reserve(xyf.size() * sizeof(float)));
+  CTSIM_HIP(hipMemcpy(p.d_xy.ptr, xyf.data(), xyf.size() * sizeof(float), hipMemcpyHostToDevice));
   return CTSIM_OK;
 }
 
@@ -841,23 +846,19 @@ int bp_mixed_tiles(ctsim_ctx* ctx, const BpPlan& p, const MixedShape& m, const v
   a.split = (nView + a.viewsPerGroup - 1) / a.viewsPerGroup;
   a.chunk = m.chunk < 1 ? 1 : (m.chunk > kMaxChunk ? kMaxChunk : m.chunk);
   a.center = static_cast<float>(p.iDetCenter);
-  a.F = static_cast<float>(p.F);
-  a.twoF = static_cast<float>(2 * p.F);
   a.endScale = static_cast<float>(endScale);
   a.overwrite = overwrite ? 1 : 0;
   const int gk = p.geom == GEOM_PARALLEL ? 0 : (p.geom == GEOM_EQUIANGULAR ? 1 : 2);
-  a.posScale = gk == 2 ? static_cast<float>(p.sdl / p.detInc) : static_cast<float>(1.0 / p.detInc);
   const int deg = gk == 1 ? p.atanDeg : 0;
   if (deg > 0) for (int k = 0; k <= deg; k++) a.atan[k] = p.atanCoef[k];
   else a.atan[0] = static_cast<float>(1.0 / p.detInc);
-  a.xs = p.d_xy.as<float>();
-  a.ys = p.d_xy.as<float>() + p.xs.size();
   a.vc = d_vc;
   a.coef = coef;
   a.image = d_image;
   const size_t npix = static_cast<size_t>(p.nx) * p.ny;
   const SymViews sv = views ? *views : p.cachedSym;
   const bool sym = m.sym && (views ? bp_sym_ok_for(p, m, sv) : bp_sym_ok(p, m, nView));
+  mixed_geometry(a, p, sym);
   // the mirror body: the mirror partners of these views (the cached ones
   // must be of these nView angles)
   const bool known = views || (static_cast<int>(p.cachedAngles.size()) == nView && p.cachedKind == 1);

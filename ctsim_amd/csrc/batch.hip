@@ -775,11 +775,7 @@ int batch_layout(ctsim_ctx* ctx, ctsim_batch& b) {
     a.endScale = static_cast<float>(p.rotScale);
     if (d.deg > 0) for (int j = 0; j <= d.deg; j++) a.atan[j] = p.atanCoef[j];
     else a.atan[0] = static_cast<float>(1.0 / p.detInc);
-    a.F = static_cast<float>(p.F);
-    a.twoF = static_cast<float>(2 * p.F);
-    a.posScale = d.gk == 2 ? static_cast<float>(p.sdl / p.detInc) : static_cast<float>(1.0 / p.detInc);
-    a.xs = p.d_xy.as<float>();
-    a.ys = p.d_xy.as<float>() + p.xs.size();
+    dev::mixed_geometry(a, p, d.sym);
     a.vc = sl.vc.as<ViewConstF32>();
     a.coef = sl.coef.ptr;
     a.image = b.images.empty() ? nullptr : b.images[k];

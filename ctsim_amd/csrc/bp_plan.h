@@ -90,7 +90,7 @@ struct BpPlan {
   std::vector<float> xs, ys;        // the same rounded to float (mixed path)
   // Device copies.
   DevBuf d_rphi;                    // r, phi, xd, yd, doubles
-  DevBuf d_xy;                      // xs then ys, floats
+  DevBuf d_xy;                      // xs then ys, floats; equilinear: then both in units of F and in cells
   // Launch shape.
   int tileX = 16, tileY = 16;       // pixels per block along ix, iy
   int windowF64 = 0, windowF32 = 0; // detector window per (tile, view); 0 = full row
