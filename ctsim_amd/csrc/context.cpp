@@ -103,6 +103,7 @@ void ctsim_ctx::prof_end_on(hipStream_t s) {
 
 ctsim_ctx::~ctsim_ctx() {
   for (hipEvent_t e : profEvents) (void)hipEventDestroy(e);
+  if (helixFlag) (void)hipHostFree(helixFlag);
 }
 
 using namespace ctsim;
@@ -131,6 +132,11 @@ int ctsim_ctx_create(ctsim_ctx** out, int device, void* stream) {
   c->stream = static_cast<hipStream_t>(stream);
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->numCUs = prop.multiProcessorCount;
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->helixFlag), sizeof(int), hipHostMallocDefault) != hipSuccess) {
+    c->helixFlag = nullptr;
+    delete c;
+    return fail(CTSIM_ERR_HIP, "ctsim_ctx_create: pinned memory allocation failed");
+  }
   *out = c;
   return CTSIM_OK;
 }

@@ -90,7 +90,8 @@ struct ctsim_ctx {
   // helical interpolation and half-scan feathering: the detector angles of
   // the last scan (rebuilt when geometry, nDet, detInc or SDL change) and the
   // feather's error word
-  ctsim::DevBuf helixGam, helixErr;
+  ctsim::DevBuf helixGam;
+  int* helixFlag = nullptr;  // pinned: the half-scan feathering's error flag
   int helixGeom = -1, helixNDet = 0;
   double helixDetInc = 0, helixSdl = 0;
   ctsim::DevBuf rasterTab;    // coordinates and sums of the rasteriser's last call

@@ -12,6 +12,11 @@
 // Fan angles per detector come from a host table (the reference's integer
 // detector centre; equilinear: atan(t / sdl), a derived geometry the
 // reference does not implement).  Arithmetic is FP64 without contraction.
+//
+// What bounds the kernels: their start and end, once the FP64 divisions are few:
+// two candidate views instead of five, the rounded views by a reciprocal
+// (conjugate_view).  At 888 detectors and 1152 views a turn 10.3 us, now 8.4,
+// and 6.7 us, now 5.9.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -26,7 +31,7 @@ namespace {
 
 struct HelixArgs {
   int nDet, nView, L, offsetView;
-  double dbeta, fan;
+  double dbeta, rdbeta, fan;  // rdbeta: 1 / dbeta
   const double* gam;  // fan angle per detector
   const float* in;    // [nView][nDet]
   float* out;         // [L+1][nDet]
@@ -34,6 +39,17 @@ struct HelixArgs {
 
 __device__ __forceinline__ int nearest_i(double x) {
   return x > 0 ? static_cast<int>(x + 0.5) : static_cast<int>(x - 0.5);
+}
+
+// The conjugate view of view iView at fan angle gamma, rounded: nearest_i of
+// ((iView dbeta) + 2 gamma - PI) / dbeta.  The quotient is formed by the
+// reciprocal, and by the reference's division only where that may round to
+// another view (both are within 1e-15 of the terms' sizes).
+__device__ __forceinline__ int conjugate_view(int iView, double gamma, double dbeta, double rdbeta) {
+  const double t = (2 * gamma - kPi) * rdbeta, u = iView + t;
+  const int n = nearest_i(u);
+  if (fabs(u - n) < 0.5 - 1e-6 - 1e-14 * (iView + fabs(t))) return n;
+  return nearest_i(((iView * dbeta) + 2 * gamma - kPi) / dbeta);
 }
 
 // Weight of an acquired sample (beta, gamma) in the reference's region chain
@@ -59,9 +75,9 @@ __device__ __forceinline__ bool region_weight(double beta, double gamma, double 
 }
 
 __global__ __launch_bounds__(256) void helical_kernel(HelixArgs a) {
-  const size_t k = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (k >= static_cast<size_t>(a.L + 1) * a.nDet) return;
-  const int nv = static_cast<int>(k / a.nDet), nd = static_cast<int>(k % a.nDet);
+  const int nv = blockIdx.x, nd = blockIdx.y * 256 + threadIdx.x;
+  if (nd >= a.nDet) return;
+  const size_t k = static_cast<size_t>(nv) * a.nDet + nd;
   const double PI = kPi, dbeta = a.dbeta, fan = a.fan;
   float acc = 0.f;
   // direct sample: acquired below pi + fan, kept in place
@@ -77,13 +93,15 @@ __global__ __launch_bounds__(256) void helical_kernel(HelixArgs a) {
   {
     const int iDet = a.nDet - 1 - nd;
     const double gamma = a.gam[iDet];
-    const double x0 = nv - (2 * gamma - PI) / dbeta;
+    // x0 is the source view that lands on nv exactly; the views that round to
+    // nv lie within a half of it, its rounding included (|x0| is below 2^31)
+    const double x0 = nv - (2 * gamma - PI) * a.rdbeta;
     const int c0 = static_cast<int>(floor(x0));
-    for (int iView = c0 - 2; iView <= c0 + 2; iView++) {
+    for (int iView = c0; iView <= c0 + 1; iView++) {
       if (iView < 0 || iView > 2 * a.L) continue;
       const double beta = iView * dbeta;
       if (beta < PI + fan) continue;
-      if (nearest_i(((iView * dbeta) + 2 * gamma - PI) / dbeta) != nv) continue;
+      if (conjugate_view(iView, gamma, dbeta, a.rdbeta) != nv) continue;
       if (iView + a.offsetView >= a.nView) continue;
       double w;
       if (region_weight(beta, gamma, fan, w))
@@ -95,7 +113,7 @@ __global__ __launch_bounds__(256) void helical_kernel(HelixArgs a) {
 
 struct FeatherArgs {
   int nDet, nView;
-  double dbeta, fan, scale;
+  double dbeta, rdbeta, fan, scale;
   const double* gam;
   const float* in;
   float* out;
@@ -118,18 +136,18 @@ __device__ __forceinline__ bool feather_x(double beta1, double gamma1, double fa
 }
 
 __global__ __launch_bounds__(256) void feather_kernel(FeatherArgs a) {
-  const size_t k = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (k >= static_cast<size_t>(a.nView) * a.nDet) return;
-  const int iv = static_cast<int>(k / a.nDet), id = static_cast<int>(k % a.nDet);
+  const int iv = blockIdx.x, id = blockIdx.y * 256 + threadIdx.x;
+  if (id >= a.nDet) return;
+  const size_t k = static_cast<size_t>(iv) * a.nDet + id;
   const double PI = kPi, dbeta = a.dbeta, fan = a.fan;
   float v = a.in[k];
   const double gamma = a.gam[id];
   if (iv * dbeta >= PI - 2 * gamma) {
     // redundant sample: keeps w2 of itself
-    const int iView1 = nearest_i(((iv * dbeta) + 2 * gamma - PI) / dbeta);
+    const int iView1 = conjugate_view(iv, gamma, dbeta, a.rdbeta);
     double x;
     if (!feather_x(iView1 * dbeta, -gamma, fan, x)) {
-      atomicOr(a.error, 1);
+      *a.error = 1;
     } else {
       const double w1 = (3 * x - 2 * x * x) * x;
       const double w2 = 1 - w1;
@@ -140,15 +158,15 @@ __global__ __launch_bounds__(256) void feather_kernel(FeatherArgs a) {
     // the last one in the reference's loop order wins (a copy, then w1)
     const int iDet2 = a.nDet - 1 - id;
     const double gamma2 = a.gam[iDet2];
-    const double x0 = iv - (2 * gamma2 - PI) / dbeta;
+    const double x0 = iv - (2 * gamma2 - PI) * a.rdbeta;
     const int c0 = static_cast<int>(floor(x0));
-    for (int iView2 = c0 - 2; iView2 <= c0 + 2; iView2++) {
+    for (int iView2 = c0; iView2 <= c0 + 1; iView2++) {
       if (iView2 < 0 || iView2 >= a.nView) continue;
       if (!(iView2 * dbeta >= PI - 2 * gamma2)) continue;
-      if (nearest_i(((iView2 * dbeta) + 2 * gamma2 - PI) / dbeta) != iv) continue;
+      if (conjugate_view(iView2, gamma2, dbeta, a.rdbeta) != iv) continue;
       double x;
       if (!feather_x(iv * dbeta, -gamma2, fan, x)) {
-        atomicOr(a.error, 1);
+        *a.error = 1;
         continue;
       }
       const double w1 = (3 * x - 2 * x * x) * x;
@@ -221,10 +239,8 @@ int ctsim_helical180li(ctsim_ctx* ctx, int geometry, int nDet, int nView, double
   CTSIM_CHECK(ctx->activate());
   const double* gam = nullptr;
   CTSIM_CHECK(gamma_table(ctx, geometry, nDet, detInc, sourceDetectorLength, &gam));
-  HelixArgs a{nDet, nView, L, offsetView, dbeta, fan, gam, d_in, d_out};
-  const size_t n = static_cast<size_t>(L + 1) * nDet;
-  hipLaunchKernelGGL(helical_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                     ctx->stream, a);
+  HelixArgs a{nDet, nView, L, offsetView, dbeta, 1.0 / dbeta, fan, gam, d_in, d_out};
+  hipLaunchKernelGGL(helical_kernel, dim3(L + 1, (nDet + 255) / 256), dim3(256), 0, ctx->stream, a);
   CTSIM_HIP(hipGetLastError());
   *nViewOut = L + 1;
   if (h_anglesOut)
@@ -245,19 +261,16 @@ int ctsim_halfscan_feather(ctsim_ctx* ctx, int geometry, int nDet, int nView, do
   CTSIM_CHECK(ctx->activate());
   const double* gam = nullptr;
   CTSIM_CHECK(gamma_table(ctx, geometry, nDet, detInc, sourceDetectorLength, &gam));
-  CTSIM_CHECK(ctx->helixErr.reserve(sizeof(int)));
-  int zero = 0;
-  CTSIM_HIP(hipMemcpyAsync(ctx->helixErr.ptr, &zero, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-  FeatherArgs a{nDet, nView, rotInc, fanBeamAngle, nView * rotInc / PI, gam, d_in, d_out,
-                ctx->helixErr.as<int>()};
-  const size_t n = static_cast<size_t>(nView) * nDet;
-  hipLaunchKernelGGL(feather_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                     ctx->stream, a);
+  // the flag lies in host memory (every call waits for the stream, so it is
+  // this call's): a copy to clear it and one to read it took 10 us of the 53 of
+  // an interpolation and a feathering of 888 detectors, 1152 views a turn
+  *ctx->helixFlag = 0;
+  FeatherArgs a{nDet, nView, rotInc, 1.0 / rotInc, fanBeamAngle, nView * rotInc / PI, gam, d_in, d_out,
+                ctx->helixFlag};
+  hipLaunchKernelGGL(feather_kernel, dim3(nView, (nDet + 255) / 256), dim3(256), 0, ctx->stream, a);
   CTSIM_HIP(hipGetLastError());
-  int flag = 0;
-  CTSIM_HIP(hipMemcpyAsync(&flag, ctx->helixErr.ptr, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   CTSIM_HIP(hipStreamSynchronize(ctx->stream));
-  if (flag) return fail(CTSIM_ERR_INVALID, "HalfScanFeather: sample outside every weighting region");
+  if (*ctx->helixFlag) return fail(CTSIM_ERR_INVALID, "HalfScanFeather: sample outside every weighting region");
   return CTSIM_OK;
 }
 
