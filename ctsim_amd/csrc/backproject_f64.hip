@@ -134,6 +134,17 @@ __device__ __noinline__ float fan_exact(double r, double phi, double theta, doub
 
 // ------------------------------------------------------------------ the kernel
 
+// The largest of non-negative numbers, less 2^-20 of it at most (which the
+// bounds' quarter covers); infinite or no number if one of them is (fmax would
+// drop the latter).  Their order is that of their high words.
+__device__ __forceinline__ unsigned high_word(double x) {
+  return static_cast<unsigned>(__builtin_bit_cast(unsigned long long, x) >> 32);
+}
+__device__ __forceinline__ double largest(double a, double b, double c, double d = 0.0) {
+  const unsigned h = max(max(high_word(a), high_word(b)), max(high_word(c), high_word(d)));
+  return __builtin_bit_cast(double, static_cast<unsigned long long>(h) << 32);
+}
+
 // Coefficients of detector interval i of row Y: on [i, i + 1) the
 // interpolant is a0 + u (a1 + u (a2 + u a3)).  Outside the detector every
 // coefficient is -0.0: adding -0.0 leaves any v as it is, and the bounds on a
@@ -142,7 +153,8 @@ __device__ __noinline__ float fan_exact(double r, double phi, double theta, doub
 // interpolant is continuous, so a position in doubt by less than a cell moves
 // the value by no more than that times the doubt), plus kappa times the
 // largest cell, which covers the coefficients' rounding; infinite beside the
-// detector's ends, where the interpolant jumps to zero.
+// detector's ends, where the interpolant jumps to zero, and infinite or no
+// number beside a cell that is, which a neighbouring interval may add.
 template <int INTERP>
 struct FanCell {  // the cubic's coefficients, or the line's two, and the slope bound
   static constexpr int kSlope = INTERP == INTERP_CUBIC ? 4 : 2;
@@ -154,12 +166,12 @@ __device__ __forceinline__ void fan_coef(double ym, double y0, double y1, double
                                          int n, double kappa, FanCell<INTERP>* cell) {
   const bool in = i >= 0 && i + 2 <= n;  // the intervals [0, n - 1)
   const double d0 = fabs(y1 - y0), d1 = fabs(y2 - y1), d2 = fabs(y3 - y2);
-  const double big = fmax(fmax(fabs(y0), fabs(y1)), fmax(fabs(y2), fabs(y3)));
+  const double big = largest(fabs(y0), fabs(y1), fabs(y2), fabs(y3));
   double slope;
   double2* out = reinterpret_cast<double2*>(cell->v);
   if constexpr (INTERP == INTERP_LINEAR) {
     out[0] = make_double2(in ? y1 : -0.0, in ? y2 - y1 : -0.0);
-    slope = fma(kappa, big, fmax(d0, fmax(d1, d2)));
+    slope = fma(kappa, big, largest(d0, d1, d2));
   } else {
     const double third = 1. / 3, sixth = 1. / 6;
     const bool interior = i > 0 && i + 2 < n;  // else (in) the first or last interval: a line
@@ -172,7 +184,7 @@ __device__ __forceinline__ void fan_coef(double ym, double y0, double y1, double
     // of its three steps' sizes (the end intervals' lines: 1 of theirs)
     const double dm = fabs(y0 - ym), dp = fabs(yp - y3), m = 1.0834;
     const double s0 = fma(m, d0, third * (dm + d1)), s1 = fma(m, d1, third * (d0 + d2)), s2 = fma(m, d2, third * (d1 + dp));
-    slope = fma(kappa, big, fmax(s1, fmax(s0, s2)));
+    slope = fma(kappa, big, largest(s0, s1, s2));
   }
   if ((i >= -1 && i <= 0) || (i >= n - 2 && i <= n - 1)) slope = __builtin_inf();
   if (i < -1 || i > n - 1) slope = 0.0;

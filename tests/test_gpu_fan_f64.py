@@ -108,3 +108,37 @@ def test_views_in_parts_add_up(gpu_ctx):
     b.backproject(rows[61:].contiguous(), angles[61:], parts, ctsim_amd.PREC_F64)
     torch.cuda.synchronize()
     assert torch.equal(whole.view(torch.int32), parts.view(torch.int32))
+
+
+@pytest.mark.parametrize("interp", ["linear", "cubic"])
+@pytest.mark.parametrize("geom", ["equiangular", "equilinear"])
+@pytest.mark.parametrize("nx", [45, 64, 129])
+def test_no_number_beside_a_cell_boundary(gpu_ctx, oracle_lib, geom, interp, nx):
+    """Views at multiples of 45 degrees put a square image's middle row,
+    column or diagonal on the centre cell to within rounding, so that the
+    reference reads either of two intervals there: a cell that is no number
+    in the one beside the interval of the short formula's position reaches the
+    pixel or not as the reference's own operations decide."""
+    import torch
+    import ctsim_amd
+    nDet = 67
+    print(f"case fan f64 no number beside a boundary {geom} {interp} {nx}", flush=True)
+    phm, scan = _scan(oracle_lib, geom, nDet, 1)
+    b = _plan(gpu_ctx, geom, nDet, 1, nx, nx, interp, _info(geom, nDet, 1))
+    row = np.random.default_rng(nx).standard_normal((1, nDet))
+    seen = 0
+    for k in range(8):  # a view at a time (a pixel that is no number stays so), some after whole turns
+        angle = np.array([(k + 8 * (k % 4)) * (np.pi / 4)])
+        for off in (-3, -2, -1, 0, 1, 2, 3):
+            bad = row.copy()
+            bad[0, (nDet - 1) // 2 + off] = np.nan
+            want = oracle_lib.backproject("oracle", phm, scan, "idiff", interp, nx, nx, bad, angle)
+            img = torch.zeros((nx, nx), dtype=torch.float32, device="cuda")
+            b.backproject(torch.from_numpy(bad).cuda(), angle, img, ctsim_amd.PREC_F64)
+            b.postprocess(img)
+            torch.cuda.synchronize()
+            out, nan = img.cpu().numpy(), np.isnan(want)
+            seen += int(nan.sum())
+            assert np.array_equal(nan, np.isnan(out)), f"view {k} cell {off}: {int((nan != np.isnan(out)).sum())} pixels"
+            assert np.array_equal(out[~nan].view(np.uint32), want[~nan].view(np.uint32)), f"view {k} cell {off}"
+    assert seen > 0
