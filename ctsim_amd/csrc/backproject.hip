@@ -381,7 +381,7 @@ template <int GK, int INTERP, int P, int DEG>
 __global__ __launch_bounds__(256) void bp_mixed_kernel(MixedArgs a) {
   extern __shared__ float4 s_dyn[];
   __shared__ float4 s_v[dev::kMaxChunk + 2];
-  __shared__ int s_lo[dev::kMaxChunk];
+  __shared__ float s_sh[dev::kMaxChunk + 2];
   const int nTiles = a.tilesX * a.tilesY;
   int tile, grp;
   if ((a.split & 7) == 0) {
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256) void bp_mixed_kernel(MixedArgs a) {
     grp = bid / nTiles;
   }
   dev::bp_mixed_tile<GK, INTERP, P, DEG>(a, tile, grp, reinterpret_cast<CoefT<INTERP>*>(s_dyn), s_v,
-                                         s_lo);
+                                         s_sh);
 }
 
 // The mirror variant: one workgroup per (tile of the mirror domain, view
@@ -639,11 +639,10 @@ int bp_upload_tables(BpPlan& p) {
   }
   std::vector<float> xyf(p.xs);
   xyf.insert(xyf.end(), p.ys.begin(), p.ys.end());
-  if (p.geom == GEOM_EQUILINEAR)  // and in units of the focal length, in detector cells at the centre
-    for (double scale : {1.0, p.sdl / p.detInc}) {
-      for (double x : p.xd) xyf.push_back(static_cast<float>(x / p.F * scale));
-      for (double y : p.yd) xyf.push_back(static_cast<float>(y / p.F * scale));
-    }
+  if (p.geom == GEOM_EQUILINEAR) {
+    for (double x : p.xd) xyf.push_back(static_cast<float>(x / p.xInc));
+    for (double y : p.yd) xyf.push_back(static_cast<float>(y / p.yInc));
+  }
   CTSIM_CHECK(p.d_xy.reserve(xyf.size() * sizeof(float)));
   CTSIM_HIP(hipMemcpy(p.d_xy.ptr, xyf.data(), xyf.size() * sizeof(float), hipMemcpyHostToDevice));
   return CTSIM_OK;

@@ -98,24 +98,24 @@ __global__ __launch_bounds__(256) void batch_combine_kernel(const SliceDev* __re
 
 template <int P>
 __device__ __forceinline__ void bp_item(const MixedArgs& a, int gk, int interp, int deg, int tile, void* smem,
-                        float4* s_v, int* s_lo) {
+                        float4* s_v, float* s_sh) {
   using dev::bp_mixed_tile;
   if (interp == INTERP_CUBIC) {
     float4* w = static_cast<float4*>(smem);
-    if (gk == 0) bp_mixed_tile<0, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_lo);
-    else if (gk == 2) bp_mixed_tile<2, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 4) bp_mixed_tile<1, INTERP_CUBIC, P, 4>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 6) bp_mixed_tile<1, INTERP_CUBIC, P, 6>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 8) bp_mixed_tile<1, INTERP_CUBIC, P, 8>(a, tile, 0, w, s_v, s_lo);
-    else bp_mixed_tile<1, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_lo);
+    if (gk == 0) bp_mixed_tile<0, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_sh);
+    else if (gk == 2) bp_mixed_tile<2, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 4) bp_mixed_tile<1, INTERP_CUBIC, P, 4>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 6) bp_mixed_tile<1, INTERP_CUBIC, P, 6>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 8) bp_mixed_tile<1, INTERP_CUBIC, P, 8>(a, tile, 0, w, s_v, s_sh);
+    else bp_mixed_tile<1, INTERP_CUBIC, P, 0>(a, tile, 0, w, s_v, s_sh);
   } else {
     float2* w = static_cast<float2*>(smem);
-    if (gk == 0) bp_mixed_tile<0, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_lo);
-    else if (gk == 2) bp_mixed_tile<2, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 4) bp_mixed_tile<1, INTERP_LINEAR, P, 4>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 6) bp_mixed_tile<1, INTERP_LINEAR, P, 6>(a, tile, 0, w, s_v, s_lo);
-    else if (deg == 8) bp_mixed_tile<1, INTERP_LINEAR, P, 8>(a, tile, 0, w, s_v, s_lo);
-    else bp_mixed_tile<1, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_lo);
+    if (gk == 0) bp_mixed_tile<0, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_sh);
+    else if (gk == 2) bp_mixed_tile<2, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 4) bp_mixed_tile<1, INTERP_LINEAR, P, 4>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 6) bp_mixed_tile<1, INTERP_LINEAR, P, 6>(a, tile, 0, w, s_v, s_sh);
+    else if (deg == 8) bp_mixed_tile<1, INTERP_LINEAR, P, 8>(a, tile, 0, w, s_v, s_sh);
+    else bp_mixed_tile<1, INTERP_LINEAR, P, 0>(a, tile, 0, w, s_v, s_sh);
   }
 }
 
@@ -295,7 +295,7 @@ __device__ __forceinline__ void fbp_batch_body(const SliceDev* __restrict__ slic
   static_assert(sizeof(dev::SymWin) == 16, "window record is one float4");
   constexpr int kMeta = SYM ? 288 : dev::kMaxChunk + 2;
   __shared__ float4 s_meta[kMeta];
-  __shared__ int s_lo[dev::kMaxChunk];
+  __shared__ float s_sh[dev::kMaxChunk + 2];
   __shared__ int s_item;
   float4* s_v = s_meta;
   dev::SymWin* s_win = reinterpret_cast<dev::SymWin*>(s_meta);
@@ -359,12 +359,12 @@ __device__ __forceinline__ void fbp_batch_body(const SliceDev* __restrict__ slic
           if (s.interp == INTERP_CUBIC) bp_sym_interp<P, INTERP_CUBIC>(s, it.a, it.pad, smem, s_ab, s_win);
           else bp_sym_interp<P, INTERP_LINEAR>(s, it.a, it.pad, smem, s_ab, s_win);
         } else {
-          bp_item<P>(s.bp, s.gk, s.interp, s.deg, it.a, smem, s_v, s_lo);
+          bp_item<P>(s.bp, s.gk, s.interp, s.deg, it.a, smem, s_v, s_sh);
         }
       } else if constexpr (MIR) {
         bp_mirror_item<P>(s.bp, s.gk, s.interp, s.deg, s.mirNM, it.a);
       } else {
-        bp_item<P>(s.bp, s.gk, s.interp, s.deg, it.a, smem, s_v, s_lo);
+        bp_item<P>(s.bp, s.gk, s.interp, s.deg, it.a, smem, s_v, s_sh);
       }
     }
     __syncthreads();  // LDS is reused by the next item
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(256) void fbp_batch_plain_class_kernel(const SliceD
                                                                     int* counters, int* /*error: no waits here*/) {
   extern __shared__ float4 smem[];
   __shared__ float4 s_v[dev::kMaxChunk + 2];
-  __shared__ int s_lo[dev::kMaxChunk];
+  __shared__ float s_sh[dev::kMaxChunk + 2];
   __shared__ int s_item;
   ItemQueue<true> queue(queueStart, counters);
   while (true) {
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(256) void fbp_batch_plain_class_kernel(const SliceD
     if constexpr (NM > 1)
       dev::bp_mirror_tile<GK, INTERP, P, DEG, NM>(s.bp, it.a, 0);
     else
-      dev::bp_mixed_tile<GK, INTERP, P, DEG>(s.bp, it.a, 0, reinterpret_cast<CoefT<INTERP>*>(smem), s_v, s_lo);
+      dev::bp_mixed_tile<GK, INTERP, P, DEG>(s.bp, it.a, 0, reinterpret_cast<CoefT<INTERP>*>(smem), s_v, s_sh);
     __syncthreads();  // LDS is reused by the next item
   }
 }

@@ -316,7 +316,12 @@ MirrorViews bp_view_consts_f32(const BpPlan& p, const double* angles, int nView,
     }
     out[v].mir[0] = out[v].mir[1] = out[v].mir[2] = 0;
     out[v].order = v;
-    out[v].pad[0] = out[v].pad[1] = 0.f;
+    const bool equilinear = p.geom == GEOM_EQUILINEAR;
+    const double cells = p.sdl / (p.detInc * p.F);
+    out[v].sc[0] = equilinear ? static_cast<float>(c * cells * p.xInc) : 0.f;
+    out[v].sc[1] = equilinear ? static_cast<float>(s * cells * p.yInc) : 0.f;
+    out[v].sc[2] = equilinear ? static_cast<float>(c / p.F * p.yInc) : 0.f;
+    out[v].sc[3] = equilinear ? static_cast<float>(s / p.F * p.xInc) : 0.f;
   }
   MirrorViews mv;
   // the mirror body reflects about the centre cell, which needs 2 * centre

@@ -25,18 +25,20 @@ struct ViewConstF64 {
   double c;         // Diff: detPosColStart       IntDiff: bit pattern of int64 colStart
 };
 
-// Per-view constants of the mixed path (32 bytes).  mir: the view's partners
+// Per-view constants of the mixed path (40 bytes).  mir: the view's partners
 // under the pixel-grid mirrors of the mirror body (MirrorViews), each
 // partner view * 2 + 1 when the partner sees the mirrored pixel at the
 // reflected detector position, + 0 when at the same position.  order: the
 // mirror body takes its base views in the order vc[0].order, vc[1].order,
 // ..., which lists each view's partners next to it, so that a view group
-// holds whole orbits and reads no other group's rows.
+// holds whole orbits and reads no other group's rows.  sc (equilinear), for
+// coordinates in pixels: cos, sin in detector cells per pixel at the centre
+// along x, y, then cos, sin in units of F per pixel along y, x.
 struct ViewConstF32 {
   float ca, sa;     // parallel: cos/detInc, sin/detInc; fan: cos, sin
   int mir[3];
   int order;
-  float pad[2];
+  float sc[4];
 };
 
 // Launch shape of the mixed kernel: a workgroup of 256 lanes covers
@@ -90,7 +92,7 @@ struct BpPlan {
   std::vector<float> xs, ys;        // the same rounded to float (mixed path)
   // Device copies.
   DevBuf d_rphi;                    // r, phi, xd, yd, doubles
-  DevBuf d_xy;                      // xs then ys, floats; equilinear: then both in units of F and in cells
+  DevBuf d_xy;                      // xs then ys, floats; equilinear: then both in pixels
   // Launch shape.
   int tileX = 16, tileY = 16;       // pixels per block along ix, iy
   int windowF64 = 0, windowF32 = 0; // detector window per (tile, view); 0 = full row

@@ -140,20 +140,13 @@ struct MixedArgs {
   int domX, domY, mapO;
 };
 
-// The geometry's constants and pixel coordinates, for the symmetric body or
-// the others.
-//
-// pos_mixed takes equilinear coordinates scaled, so that a position and its
-// weight need no multiplication by sdl / detInc and F (15 operations an update
-// for 17, and with tables rounded once a smaller error against 64 bits: 2.0 for
-// 2.0e-6 at 501 x 413, 4.1 for 4.3e-6 at 768^2).  The symmetric body shares the
-// products of four members; there the scale gained no time and lost precision.
+// The geometry's constants and pixel coordinates: for the plain and mirror
+// bodies (sym: false) the equilinear ones in pixels.
 inline void mixed_geometry(MixedArgs& a, const BpPlan& p, bool sym) {
-  const size_t n = p.xs.size() + p.ys.size();
   a.F = static_cast<float>(p.F);
   a.twoF = static_cast<float>(2 * p.F);
   a.posScale = static_cast<float>(p.geom == GEOM_EQUILINEAR ? p.sdl / p.detInc : 1.0 / p.detInc);
-  a.xs = p.d_xy.as<float>() + (p.geom == GEOM_EQUILINEAR && !sym ? n : 0);
+  a.xs = p.d_xy.as<float>() + (p.geom == GEOM_EQUILINEAR && !sym ? p.xs.size() + p.ys.size() : 0);
   a.ys = a.xs + p.xs.size();
 }
 
@@ -233,66 +226,68 @@ __device__ __forceinline__ float fan_angle(const float* c, float t, float add) {
   }
 }
 
+// One view's constants of the plain and mirror bodies.  Parallel: ca, sa carry
+// 1/detInc; equiangular: cos, sin of the view angle, .w unused; both with the
+// centre minus the window's start in .z.  Equilinear: ViewConstF32::sc, the
+// centre minus the window's start beside them.
+//
+// Equilinear coordinates are in pixels, whole or half numbers in a centred
+// image, and all scales lie in the view's constants, which are rounded once in
+// any case: a position and its weight need no product with sdl / detInc and F
+// (15 operations an update for 17) and carry no rounding of the coordinates.
+// Error against 64 bits over 13 sizes from 97^2 to 768^2, three scans each: 0.73
+// to 1.00 of that with products and coordinates in units of length.
+// The symmetric body shares the products of four members; there the scale
+// gained no time.
+template <int GK>
+__device__ __forceinline__ float4 view_consts4(const ViewConstF32& c, float cshift) {
+  if constexpr (GK == 2) return make_float4(c.sc[0], c.sc[1], c.sc[2], c.sc[3]);
+  else return make_float4(c.ca, c.sa, cshift, 0.f);
+}
+
 // Position of pixel (x, y) in one view (window-relative when cshift is the
-// centre minus the window start) and its weight.  Parallel: ca, sa carry
-// 1/detInc.  Fan: ca, sa = cos, sin of the view angle.
+// centre minus the window start) and its weight.  r2mF2 (equiangular): r^2 - F^2.
 template <int GK, int DEG>
-__device__ __forceinline__ void pos_mixed(const MixedArgs& a, float ca, float sa, float cshift,
-                                          float x, float y, float xe, float e, float& pos, float& wgt) {
+__device__ __forceinline__ void pos_mixed(const MixedArgs& a, const float4& c, float cshift, float x, float y,
+                                          float r2mF2, float& pos, float& wgt) {
   if constexpr (GK == 0) {
-    pos = fmaf(y, sa, fmaf(x, ca, cshift));
+    pos = fmaf(y, c.y, fmaf(x, c.x, cshift));
     wgt = 1.f;
   } else {
-    // the x terms are common to a lane's rows: x ca and F + x sa once per view
-    const float fl = fmaf(-y, ca, fmaf(x, sa, GK == 2 ? 1.f : a.F));  // F + r sin(beta - phi)
+    // the x terms are common to a lane's rows, once per view
+    const float rc = fmaf(y, c.y, x * c.x);  // r cos(beta - phi)
     if constexpr (GK == 1) {
-      const float rc = fmaf(y, sa, x * ca);  // r cos(beta - phi)
+      const float fl = fmaf(-y, c.x, fmaf(x, c.y, a.F));  // F + r sin(beta - phi)
       // one reciprocal for both 1/fl and 1/L^2, L^2 = fl^2 + rc^2 = 2 F fl + r^2 - F^2
-      const float L2 = fmaf(a.twoF, fl, e);
+      const float L2 = fmaf(a.twoF, fl, r2mF2);
       const float rr = __builtin_amdgcn_rcpf(fl * L2);
       pos = fan_angle<DEG>(a.atan, rc * (L2 * rr), cshift);
       wgt = fl * rr;
     } else {
-      // x, y in units of F; xe, e in detector cells at the centre
-      const float q = __builtin_amdgcn_rcpf(fl);
-      pos = fmaf(fmaf(e, sa, xe * ca), q, cshift);
+      const float q = __builtin_amdgcn_rcpf(fmaf(-y, c.z, fmaf(x, c.w, 1.f)));
+      pos = fmaf(rc, q, cshift);
       wgt = q * q;
     }
   }
 }
 
-// pos_mixed's xe and e for a tile's corner (equiangular: e = r^2 - F^2).
 template <int GK>
-__device__ __forceinline__ float corner_xe(const MixedArgs& a, float x) {
-  return GK == 2 ? x * a.posScale : x;
-}
-template <int GK>
-__device__ __forceinline__ float corner_e(const MixedArgs& a, float x, float y) {
-  return GK == 2 ? y * a.posScale : fmaf(x, x, fmaf(y, y, -a.F * a.F));
-}
-// ... and for a lane's column ix and row iy, the equilinear ones from the table
-// after xs, ys (rounded once).
-template <int GK>
-__device__ __forceinline__ float col_xe(const MixedArgs& a, int ix, float x) {
-  return GK == 2 ? a.xs[a.nx + a.ny + ix] : x;
-}
-template <int GK>
-__device__ __forceinline__ float row_e(const MixedArgs& a, float x, int iy, float y) {
-  return GK == 2 ? a.ys[a.nx + a.ny + iy] : corner_e<GK>(a, x, y);
+__device__ __forceinline__ float r2mF2_of(const MixedArgs& a, float x, float y) {
+  return GK == 1 ? fmaf(x, x, fmaf(y, y, -a.F * a.F)) : 0.f;
 }
 
 // One workgroup's work item: a tile of (256 / lanesY) columns x
-// (lanesY * P) rows and one group of views.  s_v must hold kMaxChunk + 2
-// entries.  Lane (cx, ly) owns column ix0 + cx and rows
-// iy0 + P*ly .. + P-1 (contiguous, so the final read-modify-write is a
-// vector access).  Per chunk of views: lanes < nv compute each view's window
-// start from the tile corners, the workgroup stages the window's interval
-// coefficients in LDS, then every lane walks the chunk's views for its P
-// pixels, summing the chunk in FP32 and folding the chunk sum into a
-// Kahan-compensated total.
+// (lanesY * P) rows and one group of views.  s_v and s_sh (the centre minus
+// the window's start) must hold kMaxChunk + 2 entries.  Lane (cx, ly) owns
+// column ix0 + cx and rows iy0 + P*ly .. + P-1 (contiguous, so the final
+// read-modify-write is a vector access).  Per chunk of views: lanes < nv
+// compute each view's window start from the tile corners, the workgroup stages
+// the window's interval coefficients in LDS, then every lane walks the chunk's
+// views for its P pixels, summing the chunk in FP32 and folding the chunk sum
+// into a Kahan-compensated total.
 template <int GK, int INTERP, int P, int DEG>
 __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int grp,
-                                              CoefT<INTERP>* s_w, float4* s_v, int* s_lo) {
+                                              CoefT<INTERP>* s_w, float4* s_v, float* s_sh) {
   using CT = CoefT<INTERP>;
   const int t = threadIdx.x;
   const int tx = 256 / a.lanesY, ty = a.lanesY * P;
@@ -301,12 +296,11 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
   const int cx1 = min(ix0 + tx - 1, a.nx - 1), cy1 = min(iy0 + ty - 1, a.ny - 1);
   const int W = a.W;
   const float x = a.xs[min(ix, a.nx - 1)];
-  const float xe = col_xe<GK>(a, min(ix, a.nx - 1), x);
-  float y[P], e[P];
+  float y[P], r2mF2[P];
 #pragma unroll
   for (int k = 0; k < P; k++) {
     y[k] = a.ys[min(iyb + k, a.ny - 1)];
-    e[k] = row_e<GK>(a, x, min(iyb + k, a.ny - 1), y[k]);
+    r2mF2[k] = r2mF2_of<GK>(a, x, y[k]);
   }
   const int vBegin = grp * a.viewsPerGroup;
   const int vEnd = min(a.nView, vBegin + a.viewsPerGroup);
@@ -323,16 +317,18 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
       if (a.W < a.nDet + 4) {
         float p0, p1, p2, p3, wd;
         const float xa = a.xs[ix0], xb = a.xs[cx1], ya = a.ys[iy0], yb = a.ys[cy1];
-        pos_mixed<GK, DEG>(a, c.ca, c.sa, a.center, xa, ya, corner_xe<GK>(a, xa), corner_e<GK>(a, xa, ya), p0, wd);
-        pos_mixed<GK, DEG>(a, c.ca, c.sa, a.center, xb, ya, corner_xe<GK>(a, xb), corner_e<GK>(a, xb, ya), p1, wd);
-        pos_mixed<GK, DEG>(a, c.ca, c.sa, a.center, xa, yb, corner_xe<GK>(a, xa), corner_e<GK>(a, xa, yb), p2, wd);
-        pos_mixed<GK, DEG>(a, c.ca, c.sa, a.center, xb, yb, corner_xe<GK>(a, xb), corner_e<GK>(a, xb, yb), p3, wd);
+        const float4 cv = view_consts4<GK>(c, a.center);
+        pos_mixed<GK, DEG>(a, cv, a.center, xa, ya, r2mF2_of<GK>(a, xa, ya), p0, wd);
+        pos_mixed<GK, DEG>(a, cv, a.center, xb, ya, r2mF2_of<GK>(a, xb, ya), p1, wd);
+        pos_mixed<GK, DEG>(a, cv, a.center, xa, yb, r2mF2_of<GK>(a, xa, yb), p2, wd);
+        pos_mixed<GK, DEG>(a, cv, a.center, xb, yb, r2mF2_of<GK>(a, xb, yb), p3, wd);
         float pmin = fminf(fminf(p0, p1), fminf(p2, p3));
         if (!(pmin > -1e9f && pmin < 1e9f)) pmin = 0.f;
         lo = static_cast<int>(floorf(pmin)) - 2;
       }
-      s_lo[t] = lo;
-      s_v[t] = make_float4(c.ca, c.sa, a.center - static_cast<float>(lo), 0.f);
+      const float cshift = a.center - static_cast<float>(lo);
+      s_sh[t] = cshift;
+      s_v[t] = view_consts4<GK>(c, cshift);
     }
     __syncthreads();
     // stage the windows, four views and two cells per lane at a time (eight
@@ -344,7 +340,7 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
         for (int u = 0; u < 4; u++) {
           const int vv = vq + u;
           const RowLoad<CT> row(coef, static_cast<size_t>(v0 + min(vv, nv - 1)) * a.nDet, vv < nv ? a.nDet : 0);
-          const int lo = s_lo[min(vv, nv - 1)];
+          const int lo = static_cast<int>(a.center - s_sh[min(vv, nv - 1)]);  // (whole numbers)
           val[u][0] = row(lo + jb + t);
           val[u][1] = row(lo + jb + t + 256);
         }
@@ -365,11 +361,14 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
     // window reads, then all interpolations), so 2P independent LDS reads are
     // in flight together; the next pair's constants are read ahead (s_v holds
     // kMaxChunk + 2 entries, so the read-ahead stays in bounds).
+    auto shift = [&](int vv, const float4& c) { return GK == 2 ? s_sh[vv] : c.z; };
     float4 c0 = s_v[0], c1 = s_v[1];
+    float h0 = shift(0, c0), h1 = shift(1, c1);
     const float wmax = static_cast<float>(W - 1);
     int vv = 0;
     for (; vv + 1 < nv; vv += 2) {
       const float4 n0 = s_v[vv + 2], n1 = s_v[vv + 3];
+      const float m0 = shift(vv + 2, n0), m1 = shift(vv + 3, n1);
       float u[2 * P], wg[2 * P];
       int j[2 * P];
 #pragma unroll
@@ -378,7 +377,7 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
 #pragma unroll
         for (int k = 0; k < P; k++) {
           float pos;
-          pos_mixed<GK, DEG>(a, c.x, c.y, c.z, x, y[k], xe, e[k], pos, wg[h * P + k]);
+          pos_mixed<GK, DEG>(a, c, h ? h1 : h0, x, y[k], r2mF2[k], pos, wg[h * P + k]);
           // interval index clamped in float (one med3; the clamp keeps NaN in
           // range too), truncated (non-negative), offset within the interval
           u[h * P + k] = __builtin_amdgcn_fractf(pos);
@@ -399,13 +398,15 @@ __device__ __forceinline__ void bp_mixed_tile(const MixedArgs& a, int tile, int 
       }
       c0 = n0;
       c1 = n1;
+      h0 = m0;
+      h1 = m1;
     }
     if (vv < nv) {
       const CT* w = s_w + vv * W;
 #pragma unroll
       for (int k = 0; k < P; k++) {
         float pos, wgt;
-        pos_mixed<GK, DEG>(a, c0.x, c0.y, c0.z, x, y[k], xe, e[k], pos, wgt);
+        pos_mixed<GK, DEG>(a, c0, h0, x, y[k], r2mF2[k], pos, wgt);
         const float uu = __builtin_amdgcn_fractf(pos);
         const CT qq = w[static_cast<int>(__builtin_amdgcn_fmed3f(pos, 0.f, wmax))];
         float val;
@@ -453,13 +454,14 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 // The staging buffers and view-block records of the mirror body, shared by
 // all of its instantiations in a kernel: per block of up to 64 base views,
-// the view constants (ca, sa, centre - lo) and, per window (view vv, member m) at vv * NM + m, the
+// the view constants (view_consts4) and, per window (view vv, member m) at vv * NM + m, the
 // detector cell of its slot 0 (low word) and its row * 2 + reflected (high
 // word; slot j then holds cell first + j, or first - j).  Plain arrays indexed from their own base,
 // so that the compiler can tell every LDS access's object.
 static __shared__ __attribute__((aligned(16))) unsigned char s_mirBuf0[kMirBufBytes];
 static __shared__ __attribute__((aligned(16))) unsigned char s_mirBuf1[kMirBufBytes];
 static __shared__ float4 s_mirView[64];
+static __shared__ float s_mirShift[64];  // equilinear
 static __shared__ long long s_mirSeg[64 * 4];
 // reflected flags of the block's windows: bit 4 (vv % 16) + m of word vv / 16
 static __shared__ unsigned long long s_mirRefl[4];
@@ -502,12 +504,11 @@ __device__ __forceinline__ void bp_mirror_tile(const MixedArgs& a, int tile, int
   const int cx1 = min(ix0 + tx - 1, a.domX - 1), cy1 = min(iy0 + ty - 1, a.domY - 1);
   const int W = a.W;
   const float x = a.xs[min(ix, a.domX - 1)];
-  const float xe = col_xe<GK>(a, min(ix, a.domX - 1), x);
-  float y[P], e[P];
+  float y[P], r2mF2[P];
 #pragma unroll
   for (int k = 0; k < P; k++) {
     y[k] = a.ys[min(iyb + k, a.domY - 1)];
-    e[k] = row_e<GK>(a, x, min(iyb + k, a.domY - 1), y[k]);
+    r2mF2[k] = r2mF2_of<GK>(a, x, y[k]);
   }
   const int vBegin = grp * a.viewsPerGroup;
   const int vEnd = min(a.nView, vBegin + a.viewsPerGroup);
@@ -545,14 +546,18 @@ __device__ __forceinline__ void bp_mirror_tile(const MixedArgs& a, int tile, int
       if (a.W < a.nDet + 4) {
         const float cx = (q & 1) ? a.xs[cx1] : a.xs[ix0], cy = (q & 2) ? a.ys[cy1] : a.ys[iy0];
         float pos, wd;
-        pos_mixed<GK, DEG>(a, c.ca, c.sa, a.center, cx, cy, corner_xe<GK>(a, cx), corner_e<GK>(a, cx, cy), pos, wd);
+        pos_mixed<GK, DEG>(a, view_consts4<GK>(c, a.center), a.center, cx, cy, r2mF2_of<GK>(a, cx, cy), pos, wd);
         pos = fminf(pos, __shfl_xor(pos, 1, 64));
         pos = fminf(pos, __shfl_xor(pos, 2, 64));
         if (!(pos > -1e9f && pos < 1e9f)) pos = 0.f;
         lo = static_cast<int>(floorf(pos)) - 2;
         if (!kCubic) lo &= ~1;  // pairs start at even cells (rounds down)
       }
-      if (q == 0) s_mirView[vv] = make_float4(c.ca, c.sa, a.center - static_cast<float>(lo), 0.f);
+      if (q == 0) {
+        const float cshift = a.center - static_cast<float>(lo);
+        s_mirView[vv] = view_consts4<GK>(c, cshift);
+        if constexpr (GK == 2) s_mirShift[vv] = cshift;
+      }
       if (q < NM) {
         const int e = q == 0 ? 2 * view : c.mir[q - 1];
         const unsigned first = static_cast<unsigned>((e & 1) ? twoC - 1 - lo : lo);
@@ -642,12 +647,13 @@ __device__ __forceinline__ void bp_mirror_tile(const MixedArgs& a, int tile, int
       // (a uniform index through readfirstlane and no read-ahead: no pointer
       // induction variable, whose object the compiler could not tell)
       const float4 c = s_mirView[__builtin_amdgcn_readfirstlane(b0 + vv)];
+      const float cshift = GK == 2 ? s_mirShift[__builtin_amdgcn_readfirstlane(b0 + vv)] : c.z;
       float u[P], u1[P], wg[P];
       int j[P];
 #pragma unroll
       for (int k = 0; k < P; k++) {
         float pos;
-        pos_mixed<GK, DEG>(a, c.x, c.y, c.z, x, y[k], xe, e[k], pos, wg[k]);
+        pos_mixed<GK, DEG>(a, c, cshift, x, y[k], r2mF2[k], pos, wg[k]);
         u[k] = __builtin_amdgcn_fractf(pos);
         u1[k] = 1.f - u[k];
         j[k] = static_cast<int>(__builtin_amdgcn_fmed3f(pos, 0.f, wmax));
