@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
 #include <cmath>
 #include <numeric>
 #include <vector>
@@ -35,7 +36,8 @@ struct RebinPlan {
   DevBuf d_t;       // [nDet] t of each run
   DevBuf d_angles;  // [nView] new view angles
   DevBuf d_pos;     // [nDet] new detector positions
-  DevBuf d_mid;     // [nView][nDet] float after the theta pass (rows beyond kRebinLds only)
+  DevBuf d_mid;     // [nView][nDet] float: the input of a run whose output overlaps it,
+                    // then (rows beyond kRebinLds only) the rows after the theta pass
 };
 
 // The largest i with dX >= X(i), or -1.  guess: tried first with its
@@ -205,7 +207,7 @@ int ctsim_rebin_create(ctsim_ctx* ctx, ctsim_rebin** out, int geometry, int nDet
   up(p.d_t, tRun.data(), nDet * sizeof(double));
   up(p.d_angles, p.newAngles.data(), nView * sizeof(double));
   up(p.d_pos, pos.data(), nDet * sizeof(double));
-  if (rc == CTSIM_OK && nDet > kRebinLds) rc = p.d_mid.reserve(nc * sizeof(float));
+  if (rc == CTSIM_OK) rc = p.d_mid.reserve((nDet > kRebinLds ? 2 : 1) * nc * sizeof(float));
   if (rc != CTSIM_OK) {
     delete r;
     return rc;
@@ -230,13 +232,20 @@ int ctsim_rebin_run(ctsim_ctx* ctx, ctsim_rebin* r, const float* d_in, float* d_
   if (!ctx || !r || !d_in || !d_out) return fail(CTSIM_ERR_INVALID, "ctsim_rebin_run: NULL argument");
   CTSIM_CHECK(ctx->activate());
   RebinPlan& p = r->p;
+  // a view's block reads rows that other blocks have replaced if the two overlap
+  const size_t n = static_cast<size_t>(p.nView) * p.nDet;
+  const std::less<const float*> before;
+  if (before(d_in, d_out + n) && before(d_out, d_in + n)) {
+    CTSIM_HIP(hipMemcpyAsync(p.d_mid.ptr, d_in, n * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
+    d_in = p.d_mid.as<float>();
+  }
   const RebinArgs a{d_in,
                     p.d_theta.as<double>(),
                     p.d_src.as<int>(),
                     p.d_t.as<double>(),
                     p.d_angles.as<double>(),
                     p.d_pos.as<double>(),
-                    p.d_mid.as<float>(),
+                    p.d_mid.as<float>() + n,
                     d_out,
                     p.nDet,
                     p.nView};

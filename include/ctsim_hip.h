@@ -333,7 +333,7 @@ int ctsim_halfscan_feather(ctsim_ctx* ctx, int geometry, int nDet, int nView, do
  * ParallelRaysums 1339-1469) for a fan-beam sinogram (geometry 1 or 2) with
  * the Projections header fields given and view angles h_angles (host): the
  * plan sorts the (theta, t) coordinates of every sample once; runs rebin
- * float [nView][nDet] rows on the device.  Exact (t, theta) ties, which the
+ * float [nView][nDet] rows on the device, also in place.  Exact (t, theta) ties, which the
  * reference's unstable sort leaves unordered, keep view-major order. */
 int ctsim_rebin_create(ctsim_ctx* ctx, ctsim_rebin** out, int geometry, int nDet, int nView,
                        double detStart, double detInc, double focalLength,

@@ -1,8 +1,8 @@
 """Rebinning where its kernel changes course: rows that just fit LDS and the
 first that do not, the smallest scans, more detectors than a block has lanes,
-and view angles far from evenly spaced (the guessed intervals miss).  And the
-helical interpolation over fan angles and view counts that move its rounded
-views.  Bit for bit against the oracle."""
+and view angles far from evenly spaced (the guessed intervals miss), and the output
+over the input.  And the helical interpolation over fan angles and view counts
+that move its rounded views.  Bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -28,6 +28,32 @@ def test_rebin_rows(gpu_ctx, oracle_lib, geom, nDet, nView, even):
     out = r.run(torch.from_numpy(data).cuda()).cpu().numpy()
     assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
     assert np.array_equal(r.angles, rang)
+
+
+@pytest.mark.parametrize("shift", [0, 1, -3])
+@pytest.mark.parametrize("nDet,nView", [(64, 65), (513, 400), (5121, 6)])
+def test_rebin_in_place(gpu_ctx, nDet, nView, shift):
+    """Output over the input, or `shift` rows beside it, and several runs on:
+    what two buffers give."""
+    import ctypes as C
+    import torch
+    import ctsim_amd
+    from ctsim_amd import api
+    print(f"case rebin in place {nDet}x{nView} shift {shift}", flush=True)
+    F, sdl, vd = 2.0, 4.0, 2.0
+    detInc = 2 * np.arcsin(vd / 2 / F) / nDet
+    angles = np.arange(nView) * (2 * np.pi / nView)
+    r = ctsim_amd.Rebin(gpu_ctx, 1, nDet, nView, -(nDet - 1) / 2 * detInc, detInc, F, sdl, vd, 0.0, angles)
+    buf = torch.zeros((nView + 6, nDet), dtype=torch.float32, device="cuda")
+    for seed in range(3):
+        sino = torch.from_numpy(np.random.default_rng(seed).standard_normal((nView, nDet)).astype(np.float32)).cuda()
+        want = r.run(sino)
+        src, dst = buf[3:3 + nView], buf[3 + shift:3 + shift + nView]
+        src.copy_(sino)
+        rc = api.lib.ctsim_rebin_run(gpu_ctx.handle, r.handle, C.c_void_p(src.data_ptr()), C.c_void_p(dst.data_ptr()))
+        api.check(rc, "ctsim_rebin_run")
+        torch.cuda.synchronize()
+        assert torch.equal(dst.view(torch.int32), want.view(torch.int32))
 
 
 @pytest.mark.parametrize("geom", [1, 2])
