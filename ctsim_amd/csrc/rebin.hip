@@ -36,8 +36,7 @@ struct RebinPlan {
   DevBuf d_t;       // [nDet] t of each run
   DevBuf d_angles;  // [nView] new view angles
   DevBuf d_pos;     // [nDet] new detector positions
-  DevBuf d_mid;     // [nView][nDet] float: the input of a run whose output overlaps it,
-                    // then (rows beyond kRebinLds only) the rows after the theta pass
+  DevBuf d_mid;     // [nView][nDet] float after the theta pass (two launches)
 };
 
 // The largest i with dX >= X(i), or -1.  guess: tried first with its
@@ -81,41 +80,60 @@ struct RebinArgs {
   int nDet, nView;
 };
 
-// One block per new view: every run interpolated to the view's angle
-// (projections.cpp:1285-1298), then the row of floats that leaves to the new
-// detector positions (1300-1325).
+// Run g at new view v (projections.cpp:1285-1298).  A run's angles are nearly
+// evenly spaced, so its interval is guessed from its ends.  The runs' tables lie
+// [entry][run], so that a wave's lanes, whose entries are nearly the same, read
+// adjacent runs.
+__device__ __forceinline__ float run_value(const RebinArgs& a, int g, double dX) {
+  const int nDet = a.nDet, nView = a.nView;
+  auto X = [&a, g, nDet](int i) { return a.theta[static_cast<size_t>(i) * nDet + g]; };
+  auto Y = [&a, g, nDet](int i) { return static_cast<double>(a.in[a.src[static_cast<size_t>(i) * nDet + g]]); };
+  const double x0 = X(0), x1 = X(nView - 1);
+  const float guess = static_cast<float>(dX - x0) / static_cast<float>(x1 - x0) * (nView - 1);
+  const int g0 = static_cast<int>(fminf(fmaxf(guess, 0.f), static_cast<float>(nView)));  // (no number: 0)
+  return static_cast<float>(lin_interp(X, Y, nView, dX, lower_index(X, nView, dX, g0)));
+}
+
+// A view's row of runs (positions t) at new detector position d
+// (projections.cpp:1300-1325), searched from d on.
+__device__ __forceinline__ float row_value(const RebinArgs& a, const double* t, const float* row, int d) {
+  auto X = [t](int i) { return t[i]; };
+  auto Y = [row](int i) { return static_cast<double>(row[i]); };
+  const double p = a.pos[d];
+  return static_cast<float>(lin_interp(X, Y, a.nDet, p, lower_index(X, a.nDet, p, d)));
+}
+
+// One block per new view, the row of floats between the two passes in LDS.
 //
-// What bounds it: the latency of the searches.  A run's angles are nearly
-// evenly spaced, so its interval is guessed from its ends; the detectors'
-// positions (LDS) are searched there.  The runs' tables lie [entry][run], so
-// that a wave's lanes, whose entries are nearly the same, read adjacent runs.
-// 720 views of 512 detectors: 16.1 us a call in two launches with binary
-// searches in memory and the row between them, 9.0 now (8.2 in the kernel).
-// LDS: false for rows that do not fit (they go through memory).
-template <bool LDS>
+// What bounds it: the latency of the searches.  720 views of 512 detectors:
+// 16.1 us a call in two launches with binary searches in memory and the row
+// between them, 9.0 now (8.2 in the kernel).
 __global__ __launch_bounds__(512) void rebin_kernel(RebinArgs a) {
   extern __shared__ double s_t[];
-  float* row = LDS ? reinterpret_cast<float*>(s_t + a.nDet) : a.mid + static_cast<size_t>(blockIdx.x) * a.nDet;
-  const int v = blockIdx.x, nView = a.nView, nDet = a.nDet;
+  const int v = blockIdx.x, nDet = a.nDet;
+  float* row = reinterpret_cast<float*>(s_t + nDet);
   const double dX = a.angles[v];
   for (int g = threadIdx.x; g < nDet; g += blockDim.x) {
-    auto X = [&a, g, nDet](int i) { return a.theta[static_cast<size_t>(i) * nDet + g]; };
-    auto Y = [&a, g, nDet](int i) { return static_cast<double>(a.in[a.src[static_cast<size_t>(i) * nDet + g]]); };
-    if (LDS) s_t[g] = a.t[g];
-    const double x0 = X(0), x1 = X(nView - 1);
-    const float guess = static_cast<float>(dX - x0) / static_cast<float>(x1 - x0) * (nView - 1);
-    const int g0 = static_cast<int>(fminf(fmaxf(guess, 0.f), static_cast<float>(nView)));  // (no number: 0)
-    row[g] = static_cast<float>(lin_interp(X, Y, nView, dX, lower_index(X, nView, dX, g0)));
+    s_t[g] = a.t[g];
+    row[g] = run_value(a, g, dX);
   }
   __syncthreads();
-  const double* t = LDS ? s_t : a.t;
-  for (int d = threadIdx.x; d < nDet; d += blockDim.x) {
-    auto X = [t](int i) { return t[i]; };
-    auto Y = [row](int i) { return static_cast<double>(row[i]); };
-    const double p = a.pos[d];
-    a.out[static_cast<size_t>(v) * nDet + d] =
-        static_cast<float>(lin_interp(X, Y, nDet, p, lower_index(X, nDet, p, d)));
-  }
+  for (int d = threadIdx.x; d < nDet; d += blockDim.x)
+    a.out[static_cast<size_t>(v) * nDet + d] = row_value(a, s_t, row, d);
+}
+
+// The two passes as launches of their own, a lane per value, the rows between
+// them in a.mid: for rows that do not fit LDS, for an output that overlaps the
+// input (the first pass has read it all), and where one block per view would go
+// through long rows alone (ctsim_rebin_run).
+__global__ __launch_bounds__(256) void rebin_runs_kernel(RebinArgs a) {
+  const int v = blockIdx.x, g = blockIdx.y * 256 + threadIdx.x;
+  if (g < a.nDet) a.mid[static_cast<size_t>(v) * a.nDet + g] = run_value(a, g, a.angles[v]);
+}
+__global__ __launch_bounds__(256) void rebin_rows_kernel(RebinArgs a) {
+  const int v = blockIdx.x, d = blockIdx.y * 256 + threadIdx.x;
+  const size_t row = static_cast<size_t>(v) * a.nDet;
+  if (d < a.nDet) a.out[row + d] = row_value(a, a.t, a.mid + row, d);
 }
 
 }  // namespace
@@ -207,7 +225,7 @@ int ctsim_rebin_create(ctsim_ctx* ctx, ctsim_rebin** out, int geometry, int nDet
   up(p.d_t, tRun.data(), nDet * sizeof(double));
   up(p.d_angles, p.newAngles.data(), nView * sizeof(double));
   up(p.d_pos, pos.data(), nDet * sizeof(double));
-  if (rc == CTSIM_OK) rc = p.d_mid.reserve((nDet > kRebinLds ? 2 : 1) * nc * sizeof(float));
+  if (rc == CTSIM_OK) rc = p.d_mid.reserve(nc * sizeof(float));
   if (rc != CTSIM_OK) {
     delete r;
     return rc;
@@ -232,29 +250,32 @@ int ctsim_rebin_run(ctsim_ctx* ctx, ctsim_rebin* r, const float* d_in, float* d_
   if (!ctx || !r || !d_in || !d_out) return fail(CTSIM_ERR_INVALID, "ctsim_rebin_run: NULL argument");
   CTSIM_CHECK(ctx->activate());
   RebinPlan& p = r->p;
-  // a view's block reads rows that other blocks have replaced if the two overlap
-  const size_t n = static_cast<size_t>(p.nView) * p.nDet;
-  const std::less<const float*> before;
-  if (before(d_in, d_out + n) && before(d_out, d_in + n)) {
-    CTSIM_HIP(hipMemcpyAsync(p.d_mid.ptr, d_in, n * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    d_in = p.d_mid.as<float>();
-  }
   const RebinArgs a{d_in,
                     p.d_theta.as<double>(),
                     p.d_src.as<int>(),
                     p.d_t.as<double>(),
                     p.d_angles.as<double>(),
                     p.d_pos.as<double>(),
-                    p.d_mid.as<float>() + n,
+                    p.d_mid.as<float>(),
                     d_out,
                     p.nDet,
                     p.nView};
-  const int threads = std::min(512, (p.nDet + 63) / 64 * 64);
-  if (p.nDet <= kRebinLds)
-    hipLaunchKernelGGL(rebin_kernel<true>, dim3(p.nView), dim3(threads),
+  const size_t n = static_cast<size_t>(p.nView) * p.nDet;
+  const std::less<const float*> before;
+  const bool overlap = before(d_in, d_out + n) && before(d_out, d_in + n);
+  // One launch while a block goes over its row in one or two rounds, and for
+  // longer rows where the views give every CU a block (three rounds) or two.  One
+  // / two launches: 1024 x 4 5.7 / 6.9 us, 1024 x 720 14 / 21, 1536 x 64 9.6 / 7.8,
+  // 1536 x 360 14 / 16, 2048 x 360 20 / 19, 4096 x 64 23 / 8.8, 4096 x 720 50 / 55.
+  const int rounds = (p.nDet + 511) / 512;
+  if (p.nDet <= kRebinLds && !overlap && p.nView >= std::min(2, std::max(0, rounds - 2)) * ctx->numCUs) {
+    hipLaunchKernelGGL(rebin_kernel, dim3(p.nView), dim3(std::min(512, (p.nDet + 63) / 64 * 64)),
                        p.nDet * (sizeof(double) + sizeof(float)), ctx->stream, a);
-  else
-    hipLaunchKernelGGL(rebin_kernel<false>, dim3(p.nView), dim3(threads), 0, ctx->stream, a);
+  } else {
+    const dim3 grid(p.nView, (p.nDet + 255) / 256);
+    hipLaunchKernelGGL(rebin_runs_kernel, grid, dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL(rebin_rows_kernel, grid, dim3(256), 0, ctx->stream, a);
+  }
   CTSIM_HIP(hipGetLastError());
   return CTSIM_OK;
 }

@@ -1,5 +1,5 @@
-"""Rebinning where its kernel changes course: rows that just fit LDS and the
-first that do not, the smallest scans, more detectors than a block has lanes,
+"""Rebinning where its kernels change course: rows that just fit LDS and the
+first that do not, one launch and two, the smallest scans, more detectors than a block has lanes,
 and view angles far from evenly spaced (the guessed intervals miss), and the output
 over the input.  And the helical interpolation over fan angles and view counts
 that move its rounded views.  Bit for bit against the oracle."""
@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("even", [True, False])
 @pytest.mark.parametrize("geom", [1, 2])
-@pytest.mark.parametrize("nDet,nView", [(2, 2), (3, 3), (64, 65), (513, 40), (5120, 6), (5121, 6)])
+@pytest.mark.parametrize("nDet,nView", [(2, 2), (3, 3), (64, 65), (513, 40), (1025, 6), (1025, 256), (1537, 511),
+                                        (2049, 512), (5120, 6), (5120, 512), (5121, 6)])
 def test_rebin_rows(gpu_ctx, oracle_lib, geom, nDet, nView, even):
     import torch
     import ctsim_amd
@@ -31,7 +32,7 @@ def test_rebin_rows(gpu_ctx, oracle_lib, geom, nDet, nView, even):
 
 
 @pytest.mark.parametrize("shift", [0, 1, -3])
-@pytest.mark.parametrize("nDet,nView", [(64, 65), (513, 400), (5121, 6)])
+@pytest.mark.parametrize("nDet,nView", [(64, 65), (513, 400), (2049, 512), (5121, 6)])
 def test_rebin_in_place(gpu_ctx, nDet, nView, shift):
     """Output over the input, or `shift` rows beside it, and several runs on:
     what two buffers give."""
