@@ -938,9 +938,13 @@ SliceScratch fbp_slice_scratch(const FilterPlan& f, const BpPlan& p, const Mixed
 }
 
 MixedShape fbp_slice_shape(const FilterPlan& f, const BpPlan& p, const SymViews& sv, int nView) {
-  const MixedShape m = bp_mixed_shape(p, sv, nView);
-  if (p.mixedTuned || fbp_slice_scratch(f, p, m, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES) return m;
-  return fbp_slice_scratch(f, p, p.mixed, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES ? p.mixed : m;
+  MixedShape m = bp_mixed_shape(p, sv, nView);
+  auto fits = [&](const MixedShape& s) {
+    return fbp_slice_scratch(f, p, s, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES;
+  };
+  if (p.mixedTuned || !fits(p.mixed)) return m;
+  while (m.split > 1 && !fits(m)) m.split /= 2;  // (with one group no partial images: it needs no more than the default)
+  return m;
 }
 
 // Per-view FP32 constants of a mixed launch on the device (cached by angles).

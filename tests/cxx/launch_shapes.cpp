@@ -1,0 +1,43 @@
+// Host decisions of the backprojection launches, printed for test_launch_shapes.py.
+//
+//   slice GEOMETRY NDET NVIEW NX NY METHOD INTERP: the mixed launch shape by rule
+//     and the one that a whole slice runs (kernel, rows per lane, lanes along y,
+//     view groups), its scratch, and the default shape's scratch
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "bp_plan.h"
+#include "filter_plan.h"
+
+using namespace ctsim;
+
+static int slice(char** v) {
+  const int geom = atoi(v[0]), nDet = atoi(v[1]), nView = atoi(v[2]), nx = atoi(v[3]), ny = atoi(v[4]);
+  const double d = 2 * std::sqrt(2.0), F = d, sdl = 2 * d, pi = 3.14159265358979323846;
+  const double fan = 2 * std::asin(0.5);
+  const double inc = geom == GEOM_PARALLEL ? d / nDet : (geom == GEOM_EQUILINEAR ? 2 * sdl * std::tan(fan / 2) : fan) / nDet;
+  BpPlan p;
+  if (bp_plan_init(p, geom, nDet, inc, nView, d, F, sdl, "idiff", v[6], 1, nx, ny, nullptr) != CTSIM_OK) return 1;
+  FilterPlan f;
+  if (filter_plan_init(f, "abs_hanning", v[5], 1 / inc, inc, nDet, 1.0, "frequency", "direct", 1, 1, geom, F, sdl) != CTSIM_OK)
+    return 1;
+  std::vector<double> angles(nView);
+  for (int k = 0; k < nView; k++) angles[k] = k * ((geom == GEOM_PARALLEL ? pi : 2 * pi) / nView);
+  std::vector<ViewConstF32> vc(nView);
+  const MirrorViews mv = bp_view_consts_f32(p, angles.data(), nView, vc.data());
+  SymViews sv = bp_sym_views(angles.data(), nView);
+  sv.NM = mv.NM;
+  sv.mapO = mv.mapO;
+  const MixedShape a = bp_auto_shape(p, sv, nView), b = fbp_slice_shape(f, p, sv, nView);
+  std::printf("rule %d %d %d %d slice %d %d %d %d scratch %zu default %zu\n", a.sym, a.P, a.lanesY, a.split, b.sym, b.P,
+              b.lanesY, b.split, fbp_slice_scratch(f, p, b, nView).total(), fbp_slice_scratch(f, p, p.mixed, nView).total());
+  return 0;
+}
+
+int main(int argc, char** argv) {
+  if (argc == 9 && !std::strcmp(argv[1], "slice")) return slice(argv + 2);
+  return 2;
+}

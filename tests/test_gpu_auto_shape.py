@@ -90,7 +90,7 @@ def test_region_of_interest(gpu_ctx):
 
 def test_static_scratch_takes_what_it_took(gpu_ctx):
     """A slice whose view groups' partial images exceed the static scratch
-    (8 x 9 MB) runs there, and as ctsim_fbp_slice, with one group."""
+    (8 x 9 MB) runs there, and as ctsim_fbp_slice, with fewer groups."""
     import ctypes as C
     import torch
     import ctsim_amd
