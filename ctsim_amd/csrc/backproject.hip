@@ -938,13 +938,14 @@ SliceScratch fbp_slice_scratch(const FilterPlan& f, const BpPlan& p, const Mixed
 }
 
 MixedShape fbp_slice_shape(const FilterPlan& f, const BpPlan& p, const SymViews& sv, int nView) {
-  MixedShape m = bp_mixed_shape(p, sv, nView);
-  auto fits = [&](const MixedShape& s) {
-    return fbp_slice_scratch(f, p, s, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES;
+  auto fits = [&](MixedShape m, int split) {
+    m.split = split;
+    return fbp_slice_scratch(f, p, m, nView).total() <= CTSIM_STATIC_SCRATCH_BYTES;
   };
-  if (p.mixedTuned || !fits(p.mixed)) return m;
-  while (m.split > 1 && !fits(m)) m.split /= 2;  // (with one group no partial images: it needs no more than the default)
-  return m;
+  if (p.mixedTuned || !fits(p.mixed, p.mixed.split)) return bp_mixed_shape(p, sv, nView);
+  int groups = 32;  // (one group has no partial images and needs no more than the default)
+  while (groups > 1 && !fits(p.mixed, groups)) groups /= 2;
+  return bp_auto_shape(p, sv, nView, groups);
 }
 
 // Per-view FP32 constants of a mixed launch on the device (cached by angles).

@@ -405,25 +405,35 @@ MixedShape bp_default_shape(const BpPlan& p, int numCUs) {
   return m;
 }
 
-
-// By what was measured over sizes from 128 to 2048, the three geometries and
-// both interpolations (whole slices, FFT filter):
+// Which kernel and tile, by what was measured over 224 slices of all three
+// geometries and both interpolations, 96 to 1980 pixels a side and square to
+// 1 : 19, some fifty shapes timed on each: whole slices 5 % above the fastest of
+// their shapes in the mean and 26 % at most (with the default shape 56 % in the
+// mean).  Figures in us:
 //   rotated copies (the pipelined rotational kernel): 8 lanes along y, 2 rows
-//     per lane (1 up to 128^2); against the mirror kernel 94 / 132 us
-//     (equilinear 512^2 linear), 142 / 187 (equiangular 512^2 cubic), 385 / 404
-//     (parallel 1024^2 cubic), 2250 / 2254 (parallel 2048^2 linear);
-//   mirror partners (the mirror kernel): 8 lanes, 4 rows from 640^2 with
-//     linear interpolation, else 2 (1 with 16 lanes up to 128^2); against the
-//     plain kernel at its default 83 / 127 (equiangular 401^2), 1167 / 1635
-//     (parallel 2048^2, 1441 views);
-//   neither (the plain kernel): 8 lanes, 4 rows (16 lanes, 1 row up to 192^2):
-//     17 / 41 (128^2), 31 / 35 (256^2), 109 / 134 (512^2), 403 / 555 (1024^2)
-//     against 16 lanes, 4 rows and one group below 256 views.
-// View groups: 8, one per XCD, or 16 where the tiles are few; at least 8 views
-// each (4 base views of the rotational kernel).
-MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView) {
+//     per lane (1 up to 224^2: equiangular 150^2 cubic 27.3 / 28.1); against the
+//     mirror kernel 67 / 77 (equiangular 396^2 cubic), 116 / 147 (equilinear 540^2
+//     linear); 2250 / 2254 (parallel 2048^2 linear);
+//   mirror partners (the mirror kernel), but for parallel and equilinear linear
+//     slices up to 450^2 (32 / 37 by the plain kernel, equilinear 147^2; beyond,
+//     84 / 96 the other way, 495^2): 8 lanes, 4 rows from 450^2 (linear; 105 / 113,
+//     527^2) or 600^2 (cubic; 240 / 280, equiangular 696^2; not parallel, 2285 /
+//     2167, 2048^2), else 2, with 16 lanes and 1 row up to 256^2 (46 / 49,
+//     equiangular 229^2 cubic);
+//   neither (the plain kernel): 8 lanes, 4 rows, 2 up to 128^2.
+// The shorter the windows, the less is staged for a tile: columns wider than
+// rows are high ("tall" images) take 16 lanes (equilinear 111 x 805 linear 94 / 166,
+// equiangular 158 x 611 cubic 127 / 180), and there linear interpolation gains
+// more from the plain kernel (94 / 120); rows higher than columns are wide
+// ("wide") take 8 lanes in small mirror slices too (parallel 390 x 142 cubic 40 /
+// 50; 2 rows with two members, 31 / 36, equilinear 437 x 138 linear).
+// View groups: 8, one per XCD, 16 where the tiles are few, and 32 in mirror slices
+// of few tiles and many views (equiangular 329 x 764, 1372 views 196 / 209); at
+// least 8 views each (4 base views of the rotational kernel).
+MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView, int maxGroups) {
   const bool cubic = p.interp == INTERP_CUBIC;
   const size_t npix = static_cast<size_t>(p.nx) * p.ny;
+  auto upTo = [&](size_t side) { return npix <= side * side; };
   auto side = [](int n, int t) { return (n + t - 1) / t; };
   auto shape = [&](int lanesY, int P, int sym, int chunk) {
     MixedShape m;
@@ -431,33 +441,49 @@ MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView) {
     m.W = bp_window_bound(p, 256 / lanesY, lanesY * P);
     return m;
   };
-  // groups over nx x ny pixels and `views` views, 16 below `few` tiles
-  auto groups = [&](MixedShape& m, int nx, int ny, int views, int few, int least) {
-    const int tiles = side(nx, 256 / m.lanesY) * side(ny, m.lanesY * m.P);
-    m.split = tiles < few ? 16 : 8;
-    while (m.split > 1 && views / m.split < least) m.split /= 2;
+  auto cells = [&](int lanesY, int P) {
+    const int W = bp_window_bound(p, 256 / lanesY, lanesY * P);
+    return W > 0 ? W : p.nDet + 4;
   };
-  const bool tiny = npix <= static_cast<size_t>(128) * 128;
+  // groups over nx x ny pixels and `views` views: 16 below `few` tiles, 32 below
+  // `fewer` and with 24 views each; false where maxGroups leaves less than four
+  // workgroups per CU of the more that there would be
+  auto groups = [&](MixedShape& m, int nx, int ny, int views, int few, int least, int fewer = 0) {
+    const int tiles = side(nx, 256 / m.lanesY) * side(ny, m.lanesY * m.P);
+    m.split = tiles < fewer && views >= 32 * 24 ? 32 : (tiles < few ? 16 : 8);
+    while (m.split > 1 && views / m.split < least) m.split /= 2;
+    const bool cut = m.split > maxGroups;
+    while (m.split > maxGroups) m.split /= 2;
+    return !cut || tiles * m.split >= 1024;
+  };
+  const bool tiny = upTo(128);
   if (sv.S > 0) {
-    MixedShape m = shape(8, tiny ? 1 : 2, 2, 2);
+    MixedShape m = shape(8, upTo(224) ? 1 : 2, 2, 2);
     if (bp_sym_ok_for(p, m, sv)) {
-      groups(m, p.nx / 2, p.nx / 2, nView / sv.S, 64, 4);
-      return m;
+      if (groups(m, p.nx / 2, p.nx / 2, nView / sv.S, 80, 4)) return m;
     }
   }
-  if (sv.NM >= 2) {
-    const bool rows4 = !cubic && npix >= static_cast<size_t>(640) * 640;
-    MixedShape m = tiny ? shape(16, 1, 3, 8) : shape(8, rows4 ? 4 : 2, 3, 8);
-    if (bp_mirror_chunk(p, m, sv.NM, nView) > 0) {
-      groups(m, side(p.nx, 2), sv.NM == 4 ? side(p.ny, 2) : p.ny, nView, 512, 8);
+  const bool tall = 1.2 * cells(16, 4) < cells(8, 4), wide = 1.25 * cells(8, 2) < cells(16, 2);
+  const bool cheap = !cubic && p.geom != GEOM_EQUIANGULAR && !tiny && !wide && (tall || upTo(450));
+  if (sv.NM >= 2 && !cheap) {
+    const bool rows4 = cubic ? p.geom != GEOM_PARALLEL && !upTo(600) : !upTo(450);
+    MixedShape m = tiny                          ? shape(16, 1, 3, 8)
+                   : tall                        ? shape(16, 2, 3, 8)
+                   : upTo(256) && !wide          ? shape(16, 1, 3, 8)
+                   : upTo(256) && sv.NM == 4     ? shape(8, 1, 3, 8)
+                   : rows4                       ? shape(8, 4, 3, 8)
+                                                 : shape(8, 2, 3, 8);
+    // (tall ones with windows so long that less than four are staged at a time: the
+    // plain kernel, equilinear 103 x 855 cubic 82 / 95)
+    const int staged = bp_mirror_chunk(p, m, sv.NM, nView) * sv.NM;
+    if (staged >= (tall ? 4 : 1) && groups(m, side(p.nx, 2), sv.NM == 4 ? side(p.ny, 2) : p.ny, nView, 512, 8, 150))
       return m;
-    }
   }
-  MixedShape m = npix <= static_cast<size_t>(192) * 192 ? shape(16, 1, 0, 16) : shape(8, 4, 0, 16);
-  const size_t view = static_cast<size_t>(m.W > 0 ? m.W : p.nDet + 4) * (cubic ? 16 : 8);
+  MixedShape m = tiny ? shape(8, 2, 0, 16) : (tall ? shape(16, 4, 0, 16) : shape(8, 4, 0, 16));
+  const size_t view = static_cast<size_t>(cells(m.lanesY, m.P)) * (cubic ? 16 : 8);
   while (m.chunk > 4 && m.chunk * view > static_cast<size_t>(36) * 1024) m.chunk /= 2;
   if (m.chunk * view > static_cast<size_t>(62) * 1024) return p.mixed;  // long windows: the default's staging
-  groups(m, p.nx, p.ny, nView, 1024, 8);
+  groups(m, p.nx, p.ny, nView, 160, 8);
   return m;
 }
 

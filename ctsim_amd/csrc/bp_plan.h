@@ -130,8 +130,9 @@ int bp_window_bound(const BpPlan& p, int tileX, int tileY);
 SymViews bp_sym_views(const double* angles, int nView);
 MixedShape bp_default_shape(const BpPlan& p, int numCUs);
 // The mixed launch shape of a plan that was neither tuned nor given one, for
-// views of this symmetry.
-MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView);
+// views of this symmetry, with no more than maxGroups (a power of two) view
+// groups.
+MixedShape bp_auto_shape(const BpPlan& p, const SymViews& sv, int nView, int maxGroups = 32);
 
 // Device side (backproject.hip).
 int bp_upload_tables(BpPlan& p);

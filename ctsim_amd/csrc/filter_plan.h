@@ -71,10 +71,10 @@ struct SliceScratch {
   size_t total() const { return vc + coef + rows + work + partial; }
 };
 SliceScratch fbp_slice_scratch(const FilterPlan& f, const BpPlan& p, const MixedShape& m, int nView);
-// The launch shape of one mixed slice (backproject.hip): bp_mixed_shape's, with
-// fewer view groups where that fits the slice into the static scratch and the
-// default shape would fit too, so that both slice entry points run one shape and
-// the static one takes every slice that the default fits.
+// The launch shape of one mixed slice (backproject.hip): bp_mixed_shape's, by rule
+// with no more view groups than fit the static scratch where the default shape
+// fits it, so that both slice entry points run one shape and the static one takes
+// every slice that the default fits.
 MixedShape fbp_slice_shape(const FilterPlan& f, const BpPlan& p, const SymViews& sv, int nView);
 
 }  // namespace ctsim

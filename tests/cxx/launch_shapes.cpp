@@ -2,7 +2,8 @@
 //
 //   slice GEOMETRY NDET NVIEW NX NY METHOD INTERP: the mixed launch shape by rule
 //     and the one that a whole slice runs (kernel, rows per lane, lanes along y,
-//     view groups), its scratch, and the default shape's scratch
+//     view groups), its scratch, and the default shape's scratch, then the
+//     detector windows of the rule's tile and of 8 and 16 lanes with 4 rows
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -32,8 +33,9 @@ static int slice(char** v) {
   sv.NM = mv.NM;
   sv.mapO = mv.mapO;
   const MixedShape a = bp_auto_shape(p, sv, nView), b = fbp_slice_shape(f, p, sv, nView);
-  std::printf("rule %d %d %d %d slice %d %d %d %d scratch %zu default %zu\n", a.sym, a.P, a.lanesY, a.split, b.sym, b.P,
-              b.lanesY, b.split, fbp_slice_scratch(f, p, b, nView).total(), fbp_slice_scratch(f, p, p.mixed, nView).total());
+  std::printf("rule %d %d %d %d slice %d %d %d %d scratch %zu default %zu windows %d %d %d\n", a.sym, a.P, a.lanesY, a.split, b.sym, b.P,
+              b.lanesY, b.split, fbp_slice_scratch(f, p, b, nView).total(), fbp_slice_scratch(f, p, p.mixed, nView).total(), a.W,
+              bp_window_bound(p, 32, 32), bp_window_bound(p, 16, 64));
   return 0;
 }
 

@@ -45,7 +45,10 @@ def _plans(ctx, geom, nDet, nView, nx, ny, interp, roi=None):
 SHAPES = [("fan", 183, 90, 128, 128, "whole"), ("fan", 64, 1, 16, 16, "whole"), ("fan", 200, 181, 129, 129, "whole"),
           ("fan", 300, 360, 256, 256, "back"), ("fan", 300, 362, 200, 200, "offset"), ("fan", 129, 77, 90, 41, "whole"),
           ("fan", 300, 200, 150, 150, "half"), ("fan", 257, 160, 256, 256, "shuffled"), ("fan", 700, 240, 641, 640, "whole"),
-          ("fan", 90, 500, 300, 300, "half")]
+          ("fan", 90, 500, 300, 300, "half"),
+          # tall and wide images, two and four mirrors, 16 and 32 groups; windows of most of the detector
+          ("fan", 210, 402, 40, 300, "whole"), ("fan", 210, 201, 300, 40, "whole"), ("fan", 150, 802, 300, 47, "whole"),
+          ("fan", 180, 770, 47, 210, "whole"), ("fan", 120, 403, 230, 230, "whole"), ("fan", 400, 302, 16, 700, "whole")]
 
 
 @pytest.mark.parametrize("interp", ["linear", "cubic"])

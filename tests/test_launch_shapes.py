@@ -44,3 +44,38 @@ def test_whole_slices_keep_the_rules_kernel(shapes, geom, nx, nView, method):
     assert used[3] == rule[3] or (used[3] < rule[3] and scratch <= STATIC_SCRATCH)
     if default <= STATIC_SCRATCH:
         assert scratch <= STATIC_SCRATCH
+
+
+@pytest.mark.parametrize("interp", ["linear", "cubic"])
+@pytest.mark.parametrize("geom", [0, 1, 2])
+@pytest.mark.parametrize("nx,ny,nDet,nView", [(103, 1980, 1790, 2655), (111, 805, 1141, 943), (158, 611, 1170, 1025),
+                                              (217, 1396, 1944, 2624), (96, 536, 499, 1042), (142, 714, 1150, 1182)])
+def test_tall_images_take_narrow_tiles(shapes, geom, interp, nx, ny, nDet, nView):
+    """Columns much wider than rows are high: tiles of 16 columns, whose
+    windows are the shorter ones."""
+    w = shapes("slice", geom, nDet, nView, nx, ny, "fft", interp)
+    lanes, windows = int(w[3]), list(map(int, w[15:18]))
+    full = nDet + 4
+    rule, eight, sixteen = (x if x > 0 else full for x in windows)
+    assert 1.2 * sixteen < eight
+    assert lanes == 16
+    assert rule <= sixteen
+
+
+@pytest.mark.parametrize("geom", [0, 2])
+@pytest.mark.parametrize("nx,ny,nDet,nView", [(138, 407, 567, 462), (148, 148, 316, 269), (149, 149, 319, 334),
+                                              (171, 171, 235, 442), (301, 301, 622, 730), (432, 432, 791, 515)])
+def test_small_linear_slices_take_the_plain_kernel(shapes, geom, nx, ny, nDet, nView):
+    """A parallel or equilinear linear update costs less than the mirror
+    kernel's staging on images this small."""
+    w = shapes("slice", geom, nDet, nView, nx, ny, "fft", "linear")
+    assert int(w[1]) == 0
+
+
+@pytest.mark.parametrize("nx,nView,method", [(423, 1516, "convolution")])
+def test_fewer_groups_leave_enough_workgroups(shapes, nx, nView, method):
+    """Where the static scratch leaves the mirror kernel too few workgroups,
+    the plain kernel's smaller share of the views fills the chip."""
+    w = shapes("slice", 0, 1606, nView, nx, 932, method, "linear")
+    assert int(w[1]) == 3 and int(w[6]) == 0
+    assert int(w[11]) <= STATIC_SCRATCH
