@@ -695,11 +695,7 @@ int bp_launch(ctsim_ctx* ctx, const BpPlan& p, int precision, const void* d_filt
         ctx, p, 0, h_angles, nView,
         [&](ViewConstF64* o) {
           bp_view_consts_f64(p, h_angles, nView, o);
-          p.cachedMaxAngle = 0;
-          for (int v = 0; v < nView; v++) {
-            const double m = fabs(h_angles[v]);
-            if (!(m <= p.cachedMaxAngle)) p.cachedMaxAngle = m;  // (a NaN stays)
-          }
+          p.cachedMaxAngle = bp_max_angle(h_angles, nView);
         },
         &a.vc));
     if (!inF32 && bp_fan_f64_ok(p, p.cachedMaxAngle))

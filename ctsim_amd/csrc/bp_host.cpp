@@ -251,6 +251,13 @@ void bp_view_consts_f64(const BpPlan& p, const double* angles, int nView, ViewCo
   }
 }
 
+double bp_max_angle(const double* angles, int nView) {
+  double m = 0;
+  for (int v = 0; v < nView; v++)
+    if (!(fabs(angles[v]) <= m) && m == m) m = fabs(angles[v]);
+  return m;
+}
+
 namespace {
 
 // Partners of every view under one pixel mirror (0: Y, 1: X, 2: O), as

@@ -128,6 +128,8 @@ void bp_view_consts_f64(const BpPlan& p, const double* angles, int nView, ViewCo
 MirrorViews bp_view_consts_f32(const BpPlan& p, const double* angles, int nView, ViewConstF32* out);
 int bp_window_bound(const BpPlan& p, int tileX, int tileY);
 SymViews bp_sym_views(const double* angles, int nView);
+// The largest angle in size; no number if one of them is none.
+double bp_max_angle(const double* angles, int nView);
 MixedShape bp_default_shape(const BpPlan& p, int numCUs);
 // The mixed launch shape of a plan that was neither tuned nor given one, for
 // views of this symmetry, with no more than maxGroups (a power of two) view

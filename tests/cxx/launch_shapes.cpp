@@ -4,6 +4,8 @@
 //     and the one that a whole slice runs (kernel, rows per lane, lanes along y,
 //     view groups), its scratch, and the default shape's scratch, then the
 //     detector windows of the rule's tile and of 8 and 16 lanes with 4 rows
+//   fan64 ANGLE...: the largest angle in size, and whether the FP64 fan-beam
+//     kernel's bounds cover it
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -39,7 +41,19 @@ static int slice(char** v) {
   return 0;
 }
 
+static int fan64(int n, char** v) {
+  std::vector<double> angles(n);
+  for (int k = 0; k < n; k++) angles[k] = std::atof(v[k]);
+  BpPlan p;
+  const double d = 2 * std::sqrt(2.0);
+  if (bp_plan_init(p, GEOM_EQUIANGULAR, 257, 0.004, n, d, d, 2 * d, "idiff", "linear", 1, 128, 128, nullptr) != CTSIM_OK) return 1;
+  const double m = bp_max_angle(angles.data(), n);
+  std::printf("%g %d\n", m, bp_fan_f64_ok(p, m) ? 1 : 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc > 2 && !std::strcmp(argv[1], "fan64")) return fan64(argc - 2, argv + 2);
   if (argc == 9 && !std::strcmp(argv[1], "slice")) return slice(argv + 2);
   return 2;
 }

@@ -79,3 +79,13 @@ def test_fewer_groups_leave_enough_workgroups(shapes, nx, nView, method):
     w = shapes("slice", 0, 1606, nView, nx, 932, method, "linear")
     assert int(w[1]) == 3 and int(w[6]) == 0
     assert int(w[11]) <= STATIC_SCRATCH
+
+
+@pytest.mark.parametrize("angles,largest,covered", [("0 1 -27.9 3", "27.9", 1), ("0 28", "28", 0), ("-1000 1", "1000", 0),
+                                                    ("1000 nan 1", "nan", 0), ("nan", "nan", 0), ("1 nan", "nan", 0),
+                                                    ("inf nan 2", "nan", 0), ("1 -inf", "inf", 0)])
+def test_fan_bounds_see_every_angle(shapes, angles, largest, covered):
+    """An angle that is no number hides no larger one from the FP64 fan-beam
+    kernel's condition."""
+    got = shapes("fan64", *angles.split())
+    assert got[0].lstrip("-") == largest and int(got[1]) == covered
