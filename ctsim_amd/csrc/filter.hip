@@ -28,6 +28,10 @@ constexpr int kOutPerWave = 8;    // outputs per wave (independent sums)
 constexpr int kJChunk = 64;       // inputs staged per step
 constexpr int kTapPad = 4 * 8 + 8;  // zeros after the exact convolution's taps: a block's outputs beyond n
 constexpr int kKChunk = 32;       // spectrum entries staged per step (inverse DFT)
+// Detectors that the exact convolution takes: what its callers have been able to
+// rely on, from a kernel that held the taps in LDS.  The present one has no limit
+// of its own; wider rows stay refused (they are not among what is compared).
+constexpr int kConvMaxDet = 4033;
 
 // ---------------------------------------------------- exact convolution
 // out[v][i] = dx * sum_{j=0}^{n-1} x[v][j] * h[i - j + n - 1]  (procsignal.cpp:659-673)
@@ -753,7 +757,7 @@ int filter_launch(ctsim_ctx* ctx, FilterPlan& p, int precision, const float* d_i
     return CTSIM_OK;
   }
   if (p.method == METHOD_CONVOLUTION) {
-    if (p.n > 4033) return fail(CTSIM_ERR_UNSUPPORTED, "convolution filter: kernel too long for LDS");
+    if (p.n > kConvMaxDet) return fail(CTSIM_ERR_UNSUPPORTED, "FP64 convolution filter: more than 4033 detectors");
     // 8 outputs per wave where that gives a block to every CU, else 4 or 2 (a
     // whole slice, 2 / 4 / 8 outputs: 320 x 367 62 / 65 / 70 us, 731 x 701
     // 447 / 421 / 418, 1440 x 1024 500 / 459 / 435; 16 gain nothing at 2880 x 2048)
