@@ -1008,11 +1008,12 @@ int raysum_launch(ctsim_ctx* ctx, const ScannerPlan& s, PhantomPlan& p, int prec
   const double rim = std::max({hypot(s.xs1, s.ys1), hypot(s.xs2, s.ys2), hypot(s.xd1, s.yd1), hypot(s.xd2, s.yd2),
                                s.centerDetLength});
   const bool fast = precision == CTSIM_PREC_F64 && !p.unitPulse && p.elems.size() <= 64 * kCandChunks &&
-                    p.fastR > 0 && 1.5 * rim + p.fastFar < 1e6 * p.fastMin;
+                    p.fastR > 0 && 1.5 * rim + p.fastFar < 1e6 * p.fastMin &&
+                    raysum_short_pays(s, p, iNumViews, ctx->numCUs);
   // Whole items are deferred where other types are met or a ray may end in the
   // elements' disc.
-  const bool deferItems = p.fastOthers || !(std::min(s.focalLength, s.centerDetLength) >
-                                            1.001 * (hypot(p.fastX - s.xc, p.fastY - s.yc) + p.fastR));
+  const bool deferItems = !p.fastOthers.empty() || !(std::min(s.focalLength, s.centerDetLength) >
+                                                     1.001 * (hypot(p.fastX - s.xc, p.fastY - s.yc) + p.fastR));
   CTSIM_CHECK(ctx->scratch.reserve(walkBytes + 256 + (fast ? (items + rays) * sizeof(int2) : 0)));
   int* counter = reinterpret_cast<int*>(static_cast<unsigned char*>(ctx->scratch.ptr) + walkBytes);
   WalkArgs wa{ctx->viewConsts.as<ViewEnds>(), ctx->scratch.as<double4>(), counter, iNumViews, s.nDet,

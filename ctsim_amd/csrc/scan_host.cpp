@@ -187,7 +187,8 @@ std::vector<FastElem> phantom_fast_elems(PhantomPlan& p) {
   p.fastR = 0;
   p.fastMin = 1e300;
   p.fastFar = 0;
-  p.fastOthers = false;
+  p.fastRects = false;
+  p.fastOthers.clear();
   for (size_t k = 0; k < p.elems.size(); k++) {
     const ElemGPU& e = p.elems[k];
     const ElemInfo& in = p.infos[k];
@@ -198,7 +199,7 @@ std::vector<FastElem> phantom_fast_elems(PhantomPlan& p) {
     const double reach = ellipse ? hi : sqrt(in.u * in.u + in.v * in.v);
     if (!(ellipse || e.type == PE_RECT) || !(lo > 0) || !(hi / lo < 1e4) || !(fabs(in.atten) < 1e30) ||
         (ellipse && in.nOutline < 32) || !(fabs(in.cx) + fabs(in.cy) + reach < 1e30)) {
-      p.fastOthers = true;
+      p.fastOthers.push_back(sqrt(in.u * in.u + in.v * in.v));
       continue;
     }
     for (int q = 0; q < 4; q++) f.m[q] = e.p2o[q];
@@ -218,6 +219,7 @@ std::vector<FastElem> phantom_fast_elems(PhantomPlan& p) {
       f.att = in.atten;
       f.edge = static_cast<float>(64 * u / lo);
       f.kind = 2;
+      p.fastRects = true;
     }
     const double dx = in.cx - p.fastX, dy = in.cy - p.fastY;
     p.fastR = fmax(p.fastR, sqrt(dx * dx + dy * dy) + reach);
@@ -226,6 +228,38 @@ std::vector<FastElem> phantom_fast_elems(PhantomPlan& p) {
   }
   p.fastR *= 1 + 1e-6;
   return out;
+}
+
+// Short chords first, the reference's chain for the rest, against the chain alone
+// (us), items being waves of 64 rays:
+//   ends inside the disc that holds the elements, for the detector's middle or all
+//     of it: every such ray is the chain's, 1024 x 720 with the detector at 0.9 of
+//     the radius equiangular 357 / 211, equilinear 336 / 286; on its rim
+//     equiangular 360 / 215, but equilinear 132 where the chain takes 321, parallel
+//     126 where it takes 250;
+//   parallel scans of few rays with rectangles (a ray along a side is left to the
+//     chain, whose latency then follows the short kernel's): 4 elements, 10 items
+//     38 / 23, 64 items 28 / 25, 180 items 27 / 28; 67 elements, 10 items 72 / 68,
+//     40 items 54 / 68;
+//   other elements: items that meet one are taken by the chain as a whole, and
+//     while the chip holds all items at once (16 to a CU) that takes as long as
+//     all of them: 64 ellipses and a triangle, 1920 items 200 / 164, 3960 items
+//     209 / 250.  Beyond, by the share of the items that meet one (each taken as
+//     its shadow and one item wide): 0.3 of 23040 items 342 / 466, 0.6 465 / 474
+//     (8 ellipses 313 / 386), all of them 424 / 359 (Herman's phantom).
+bool raysum_short_pays(const ScannerPlan& s, const PhantomPlan& p, int nView, int numCUs) {
+  const double disc = hypot(p.fastX - s.xc, p.fastY - s.yc) + p.fastR;
+  const double source = s.focalLength / disc, detector = s.centerDetLength / disc;
+  if (detector < (s.geom == GEOM_EQUIANGULAR ? 1.001 : 0.999) || source < (s.geom == GEOM_PARALLEL ? 0.999 : 1.001))
+    return false;
+  const int blocks = (s.nDet + 63) / 64;
+  const double items = static_cast<double>(blocks) * nView;
+  if (s.geom == GEOM_PARALLEL && p.fastRects && items * s.nSample * p.elems.size() < 500) return false;
+  if (p.fastOthers.empty()) return true;
+  if (items < 12.0 * numCUs) return false;
+  double clear = 1;
+  for (double reach : p.fastOthers) clear *= fmax(0.0, 1 - reach / p.fastR - 1.0 / blocks);
+  return 1 - clear < 0.65;
 }
 
 // Phantom::createFromPhantom, addStdHerman, addStdSheppLogan,

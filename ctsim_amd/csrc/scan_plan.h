@@ -55,7 +55,8 @@ struct PhantomPlan {
   // Of the elements with a short chord: a disc about the extent's centre that
   // holds them, the smallest semi-axis, the largest |centre| + semi-axis
   double fastX = 0, fastY = 0, fastR = 0, fastMin = 1e300, fastFar = 0;
-  bool fastOthers = false;  // there are elements without one
+  bool fastRects = false;          // there are rectangles among them
+  std::vector<double> fastOthers;  // half sizes of the elements without one
 };
 
 struct ScannerPlan {
@@ -85,6 +86,9 @@ void scanner_view_ends(const ScannerPlan& s, int iStartView, int iNumViews, int 
 
 // FastElem of every element, and the plan's summary of them.
 std::vector<FastElem> phantom_fast_elems(PhantomPlan& p);
+// Whether the short chord is worth its launches for a scan of nView views on a
+// chip of numCUs CUs, the plan's summary being there (raysum.hip runs it).
+bool raysum_short_pays(const ScannerPlan& s, const PhantomPlan& p, int nView, int numCUs);
 // Uploads the elements if they changed.
 int phantom_upload(PhantomPlan& p);
 int raysum_launch(ctsim_ctx* ctx, const ScannerPlan& s, PhantomPlan& p, int precision,

@@ -1,4 +1,4 @@
-// Host decisions of the backprojection launches, printed for test_launch_shapes.py.
+// Host decisions of the launches, printed for test_launch_shapes.py.
 //
 //   slice GEOMETRY NDET NVIEW NX NY METHOD INTERP: the mixed launch shape by rule
 //     and the one that a whole slice runs (kernel, rows per lane, lanes along y,
@@ -6,6 +6,8 @@
 //     detector windows of the rule's tile and of 8 and 16 lanes with 4 rows
 //   fan64 ANGLE...: the largest angle in size, and whether the FP64 fan-beam
 //     kernel's bounds cover it
+//   scan GEOMETRY NDET NVIEW FOCAL CENTER ELLIPSES RECTANGLES TRIANGLES SIZE (or a
+//     phantom's name): whether the short ray sums run
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -14,6 +16,7 @@
 
 #include "bp_plan.h"
 #include "filter_plan.h"
+#include "scan_plan.h"
 
 using namespace ctsim;
 
@@ -52,7 +55,32 @@ static int fan64(int n, char** v) {
   return 0;
 }
 
+static int scan(int n, char** v) {
+  PhantomPlan p;
+  if (n == 6) {
+    if (phantom_builtin(p, v[5]) != CTSIM_OK) return 1;
+  } else {
+    phantom_add(p, "rectangle", 0, 0, 1, 1, 0, 0.1);
+    unsigned seed = 1;
+    auto at = [&]() { return ((seed = seed * 1664525u + 1013904223u) >> 8) / 16777216.0 - 0.5; };
+    const char* const types[] = {"ellipse", "rectangle", "triangle"};
+    for (int t = 0; t < 3; t++)
+      for (int k = 0; k < std::atoi(v[5 + t]); k++) {
+        const double x = at(), y = at(), size = t == 2 ? std::atof(v[8]) : 0.1;
+        phantom_add(p, types[t], x, y, size, size, 360 * at(), 0.3);
+      }
+  }
+  ScannerPlan s;
+  if (scanner_init(s, p, v[0], std::atoi(v[1]), std::atoi(v[2]), 0, 1, v[0][0] == 'p' ? 3.14159265358979323846 : 6.28318530717958647692,
+                   std::atof(v[3]), std::atof(v[4]), 1, 1) != CTSIM_OK)
+    return 1;
+  phantom_fast_elems(p);
+  std::printf("%d\n", raysum_short_pays(s, p, s.nView, 256) ? 1 : 0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc >= 8 && !std::strcmp(argv[1], "scan")) return scan(argc - 2, argv + 2);
   if (argc > 2 && !std::strcmp(argv[1], "fan64")) return fan64(argc - 2, argv + 2);
   if (argc == 9 && !std::strcmp(argv[1], "slice")) return slice(argv + 2);
   return 2;

@@ -52,3 +52,28 @@ def test_raysums_match_oracle(gpu_ctx, oracle_lib, name, geom, nDet, nView, nSam
     torch.cuda.synchronize()
     assert record_parity(f"oracle short raysum {name} {geom} {nDet}x{nView}x{nSample} {focal}", sino.cpu().numpy(),
                          ref["sino"]) == 0
+
+
+# scans large enough that items which meet another type go to the chain by themselves, and scans whose rays end
+# in the disc of the elements (the detector's middle, or the rim)
+FEW_OTHERS = BOX + _ellipses(20, 8, 0.02, 0.3) + [("triangle", 0.4, 0.1, 0.03, 0.05, 20.0, 0.4)]
+
+
+@pytest.mark.parametrize("name,geom,nDet,nView,focal,center", [
+    ("others", "parallel", 130, 1100, 2.0, 2.0), ("others", "equiangular", 200, 800, 2.0, 2.0),
+    ("others", "equilinear", 191, 1030, 2.0, 2.0), ("circles", "parallel", 127, 40, 1.0, 1.0),
+    ("turned", "parallel", 200, 33, 2.0, 1.0), ("circles", "equilinear", 130, 40, 2.0, 1.0),
+    ("turned", "equilinear", 130, 40, 2.0, 0.9), ("circles", "equiangular", 130, 40, 2.0, 1.0)])
+def test_deferred_items_match_oracle(gpu_ctx, oracle_lib, name, geom, nDet, nView, focal, center):
+    import torch
+    import ctsim_amd
+    print(f"case short raysum {name} {geom} {nDet}x{nView} focal {focal} center {center}", flush=True)
+    O, elems = oracle_lib, FEW_OTHERS if name == "others" else PHANTOMS[name]
+    rot = np.pi if geom == "parallel" else 2 * np.pi
+    ref = O.pipeline("oracle", O.Phantom(None, elems), O.ScanSpec(geom, nDet, nView, 0, 1, rot, focal, center))
+    sc = ctsim_amd.Scanner(ctsim_amd.Phantom(None, elems), geom, nDet, nView, 0, 1, rot, focal, center)
+    sino = torch.zeros((nView, nDet), dtype=torch.float32, device="cuda")
+    sc.collect(gpu_ctx, sino, ctsim_amd.PREC_F64)
+    torch.cuda.synchronize()
+    assert record_parity(f"oracle short raysum {name} {geom} {nDet}x{nView} {focal} {center}", sino.cpu().numpy(),
+                         ref["sino"]) == 0

@@ -1,4 +1,4 @@
-"""Host decisions of the backprojection launches (CPU only, no kernel runs)."""
+"""Host decisions of the launches (CPU only, no kernel runs)."""
 import os
 import shutil
 import subprocess
@@ -89,3 +89,18 @@ def test_fan_bounds_see_every_angle(shapes, angles, largest, covered):
     kernel's condition."""
     got = shapes("fan64", *angles.split())
     assert got[0].lstrip("-") == largest and int(got[1]) == covered
+
+
+@pytest.mark.parametrize("args,short", [
+    ("equiangular 1024 1440 2 2 64 4 0 0", 1), ("parallel 367 320 2 2 8 2 0 0", 1), ("equiangular 33 10 2 2 8 2 0 0", 1),
+    # few parallel rays, some of them along a rectangle's side
+    ("parallel 33 10 2 2 1 2 0 0", 0), ("parallel 64 64 2 2 1 2 0 0", 0), ("parallel 33 40 2 2 64 2 0 0", 1),
+    # other types: in few of many items, in most items, in a scan that the chip holds at once
+    ("equilinear 1024 1440 2 2 64 2 1 0.1", 1), ("equilinear 1024 1440 2 2 64 2 10 0.2", 0),
+    ("equilinear 367 320 2 2 64 2 1 0.03", 0), ("equiangular 1024 1440 2 2 herman", 0),
+    ("equiangular 1024 1440 2 2 shepp-logan", 1),
+    # ends of rays in the elements' disc
+    ("equiangular 1024 720 2 1 8 2 0 0", 0), ("equilinear 1024 720 2 1 8 2 0 0", 1),
+    ("equilinear 1024 720 2 0.9 8 2 0 0", 0), ("parallel 1024 720 0.9 2 8 2 0 0", 0), ("parallel 1024 720 1 1 8 2 0 0", 1)])
+def test_short_ray_sums_where_they_pay(shapes, args, short):
+    assert shapes("scan", *args.split()) == [str(short)]
